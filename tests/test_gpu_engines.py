@@ -461,6 +461,32 @@ def test_run_3d_blast_long_segments(dev, oracle, engine, waves):
         assert_bitwise(got32[k], ref32[k], "fp32-flux " + k)
 
 
+@pytest.mark.parametrize("engine,mixed", [("roe", False), ("roe", True), ("hlld", False), ("hlld", True)])
+@pytest.mark.parametrize("shape", [(99, 97, 95), (131, 60, 41), (21, 19, 120)])
+def test_run_3d_default_segments(dev, engine, mixed, shape):
+    """The default segments of the 3D marches (the grid's own number: 8-face
+    segments and the fused Roe z march at 99x97x95, 3-face ones at 131x60x41,
+    single faces at 21x19x120) against one face per segment and the separate
+    Roe passes: the same bits."""
+    from utrip_amd import cans
+    case("run 3d default segments", engine, "fp32-flux" if mixed else "fp64", shape)
+    n = tuple(k + 6 for k in shape)
+    f = smooth_state_3d(*n, seed=11, bscale=3.0 if engine == "roe" else 0.8)
+    dx, dxm, dy, dym, dz, dzm = grid3(*n)
+    grid = dict(dx=dx, dxm=dxm, dy=dy, dym=dym, dz=dz, dzm=dzm)
+    pp = dict(gm=5.0 / 3.0, safety=0.4, dtmin=1e-10)
+    fields = {k: f[k] for k in F3}
+    got, info = run_gpu(dev, 3, engine, fields, grid, pp, 3, 7, 3, mixed=mixed)
+    cans.set_march_waves(1 << 22)
+    try:
+        ref, iref = run_gpu(dev, 3, engine, fields, grid, pp, 3, 7, 3, mixed=mixed)
+    finally:
+        cans.set_march_waves(32768)
+    assert info["nexec"] == 3 and info["dt"] == iref["dt"]
+    for k in F3:
+        assert_bitwise(got[k], ref[k], k)
+
+
 def test_march_waves_rejects_zero(dev):
     from utrip_amd import cans
     with pytest.raises(cans.CansError):

@@ -48,7 +48,8 @@ def _check(rc: int) -> None:
 
 def set_march_waves(waves: int) -> None:
     """Minimum wavefronts per launch of the marching face kernels (HLLD y/z
-    sweeps, 3D Roe y/z fluxes; default 32768): fewer waves, longer segments.
+    sweeps, 3D Roe y/z fluxes): fewer waves, longer segments.  The default,
+    32768, leaves the number to the library (from the grid's sizes).
     Results do not depend on it."""
     _check(lib().cans_gpu_set_march_waves(int(waves)))
 

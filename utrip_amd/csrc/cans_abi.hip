@@ -86,7 +86,7 @@ inline size_t al(size_t n) { return (n + 63) & ~size_t(63); }  // doubles, 512-b
 int cans::abi_scratch(size_t bytes, void **out, hipStream_t s) { return pool_scratch(bytes, out, s); }
 
 namespace {
-std::atomic<int> g_march_waves{32768};
+std::atomic<int> g_march_waves{kMarchWavesAuto};
 std::atomic<int> g_mlw3d_path{1};
 }
 int cans::march_waves() { return g_march_waves.load(); }

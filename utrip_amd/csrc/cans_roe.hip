@@ -808,8 +808,7 @@ hipError_t launch_roe_t(const RoeArgs &a, hipStream_t s) {
                 const int nf = stage == 1 ? n[2] - 1 : n[2] - 3;
                 const size_t cols = (size_t)(stage == 1 ? n[0] - 2 : n[0] - 4) *
                                     (size_t)(stage == 1 ? n[1] - 2 : n[1] - 4);
-                int nseg = (int)(((unsigned long long)march_waves() * 64 + cols - 1) / cols);
-                nseg = nseg < 1 ? 1 : (nseg > nf ? nf : nseg);
+                int nseg = march_segments(cols, nf);
                 int H = (nf + nseg - 1) / nseg;
                 H = H < 8 ? 8 : H;
                 nseg = (nf + H - 1) / H;
@@ -828,14 +827,12 @@ hipError_t launch_roe_t(const RoeArgs &a, hipStream_t s) {
             }
             if (D == 3 && dir >= 1) {   // y faces (and z faces without the fusion)
                 // y and z faces marched (roe_flux_march3: 384^3 FP64 step 26.4 ->
-                // 23.7 ms, FP32-flux 19.5 -> 17.7 ms); segments along dir so that
-                // the launch has >= march_waves() waves
+                // 23.7 ms, FP32-flux 19.5 -> 17.7 ms)
                 const int nf = stage == 1 ? n[dir] - 1 : n[dir] - 3;     // faces along dir
                 const int od = dir == 1 ? 2 : 1;
                 const size_t cols = (size_t)(stage == 1 ? n[0] - 2 : n[0] - 4) *
                                     (size_t)(stage == 1 ? n[od] - 2 : n[od] - 4);
-                int nseg = (int)(((unsigned long long)march_waves() * 64 + cols - 1) / cols);
-                nseg = nseg < 1 ? 1 : (nseg > nf ? nf : nseg);
+                int nseg = march_segments(cols, nf);
                 const int H = (nf + nseg - 1) / nseg;
                 nseg = (nf + H - 1) / H;
                 const size_t threads = cols * (size_t)nseg;
@@ -886,16 +883,15 @@ hipError_t launch_roe_t(const RoeArgs &a, hipStream_t s) {
 }  // namespace
 
 // 3D: z faces fused with the cell updates (roe_zmarch3) where the march's
-// segments come out at >= 8 faces for the launch's wave target (about 256^3
-// and up at the default); on smaller grids the segments would be a face or
-// two long and the fused march would compute most z faces twice, so they
-// take the separate passes.
+// segments (march_segments) come out at >= 8 faces, about 92^3 and up at the
+// default (FP64 step at 96^3 492 us with the separate passes and the same
+// waves, 435 fused; 192^3 3412 -> 2947); on smaller grids the segments would
+// be a face or two long and the fused march would compute most z faces
+// twice, so they take the separate passes (64^3: 209 us).
 bool roe3d_fused_z(int ix, int jx, int kx) {
     if (ix < 3 || jx < 3 || kx < 3) return false;
-    const size_t cols = (size_t)(ix - 2) * (size_t)(jx - 2);
     const int nf = kx - 1;
-    long nseg = (long)(((unsigned long long)march_waves() * 64 + cols - 1) / cols);
-    nseg = nseg < 1 ? 1 : (nseg > nf ? nf : nseg);
+    const int nseg = march_segments((size_t)(ix - 2) * (size_t)(jx - 2), nf);
     return (nf + nseg - 1) / nseg >= 8;
 }
 

@@ -96,8 +96,33 @@ hipError_t launch_hlld(const HlldArgs &a, bool mixed, hipStream_t s);
 
 // Marching face kernels (HLLD y/z sweeps, Roe 3D y/z fluxes) split each
 // column into segments so that a launch has at least this many waves
-// (default 32768; cans_gpu_set_march_waves changes it).
+// (cans_gpu_set_march_waves; at the default kMarchWavesAuto the number comes
+// from the grid, march_segments).
+constexpr int kMarchWavesAuto = 32768;
 int march_waves();
+// Segments of a column of nf faces (or cells) when `cols` columns march, a
+// thread each.  Each segment computes one face twice, so segments want to be
+// long; the chip wants waves (2048 run at a time at two per SIMD).  The rule
+// at the default: 16384 waves, but no segment shorter than 8 faces unless the
+// launch then has under 2048 waves.  Whole steps against 32768 waves at every
+// size (n^3, FP64 Roe / FP32-flux HLLD): 96: 529 -> 435 / 443 -> 356 us,
+// 128: 1107 -> 965 / 866 -> 769, 160: 2047 -> 1792 / 1425 -> 1336, 192: 3412
+// -> 2947 / 2387 -> 2240 (4-face segments before: a fifth of the faces
+// twice, and the separate Roe passes); 256: 6832 -> 6742 / 4977 -> 4917, and
+// 320^3 and 64^3 within 1 %.  16384 against 8192 at 256^3: 6742 / 6883.
+inline int march_segments(size_t cols, int nf) {
+    const auto seg_for = [cols](unsigned long long waves) { return (waves * 64 + cols - 1) / cols; };
+    unsigned long long nseg;
+    if (march_waves() == kMarchWavesAuto) {
+        const unsigned long long lng = ((unsigned long long)nf + 7) / 8, few = seg_for(2048);
+        nseg = seg_for(16384);
+        const unsigned long long cap = lng > few ? lng : few;
+        if (nseg > cap) nseg = cap;
+    } else {
+        nseg = seg_for((unsigned long long)march_waves());
+    }
+    return nseg < 1 ? 1 : (nseg > (unsigned long long)nf ? nf : (int)nseg);
+}
 // 3D MLW, Cartesian grids: 1 (default) = the z-marching kernel of
 // cans_mlw3d_march.hip, 0 = the three kernels over HBM scratch of
 // cans_mlw3d.hip (cans_gpu_set_mlw3d_path changes it).
