@@ -205,6 +205,27 @@ def sum_sequential(xs):
     return t
 
 
+@pytest.mark.parametrize("nx,ny", [(64, 61), (255, 250), (311, 401), (700, 130)])
+def test_mlw2d_resident_rows_per_wave(dev, oracle, nx, ny):
+    """Resident periodic runs on grids whose strips take 1 to 5 rows per wave
+    (one row at 64x61, a ragged last strip at the others): the state and dt
+    after 5 steps, bit for bit."""
+    from utrip_amd import cans
+    _print_case("mlw2d rows per wave", nx, ny)
+    pb = P.orszag_tang_box(nx, ny, margin=1)
+    ref, dts = _loop_2d_oracle(oracle, pb, 5)
+    g, pp = pb.grid, pb.params
+    gd = {k: to_dev(v, dev) for k, v in g.items()}
+    run = cans.MlwRun2D([to_dev(pb.fields[k], dev) for k in F2], gd["dx"], gd["dxm"], gd["dy"], gd["dym"],
+                        pp["qav"], pp["gm"], pp["safety"], margin=1)
+    run.reset(dtmin=pp["dtmin"])
+    run.steps(5)
+    cur, info = run.state()
+    assert info["nexec"] == 5 and info["dt"] == dts[-1]
+    for k, t in zip(F2, cur):
+        assert_bitwise(to_host(t), ref[k], k)
+
+
 def test_mlw2d_resident_stops_at_tend(dev, oracle):
     """t < tend loop test: steps after the end are no-ops."""
     from utrip_amd import cans

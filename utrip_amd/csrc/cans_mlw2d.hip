@@ -693,17 +693,25 @@ __global__ void batch2d_prep(Batch2dArgs b) {
 constexpr int kOcc = CANS_MLW2D_OCC;
 constexpr int kSlots = 256 * 4 * kOcc; // wave slots of the 256 CUs
 
-// Rows per wave: each wave pays about 1.5 rows of prologue, and the launch
-// runs in ceil(waves / slots) rounds, so pick H minimising rounds * (H + 1.5).
+// Rows per wave.  Each wave pays about 1.5 rows of prologue, and a row takes
+// about 2.0 us for a wave that has its SIMD to itself and 3.3 us for each of
+// two that share one (FP64 latency against FP64 issue), so the launch's cost
+// is (H + 1.5) * (3.3 per full round of 2048 waves, plus 2.0 or 3.3 for the
+// rest by whether it has more waves than SIMDs).  Small grids so take short
+// strips, many waves deep across the chip: whole steps with 8 rows at least
+// and with this rule, 64^2 22.8 -> 9.0 us (1 row), 256^2 23.2 -> 13.1 (2),
+// 512^2 23.2 -> 17.1 (5), 700^2 30.9 -> 25.9 (9), 2000x300 31.3 -> 25.7 (5);
+// 1024^2 (9 rows) and up as before.
 int pick_rows(int ix, int jx) {
     if (CANS_MLW2D_ROWS > 0) return CANS_MLW2D_ROWS;
-    const int nstrip = (ix - 2 + COLS - 1) / COLS;
+    const long nstrip = (ix - 2 + COLS - 1) / COLS;
+    constexpr double kAlone = 2.0, kShared = 3.3;   // us per row
     int best = 16;
     double cost = 1e300;
-    for (int h = 8; h <= 96; h++) {
-        const long waves = (long)nstrip * ((jx - 2 + h - 1) / h);
-        const long rounds = (waves + kSlots - 1) / kSlots;
-        const double c = (double)rounds * (h + 1.5);
+    for (int h = 1; h <= 96; h++) {
+        const long waves = nstrip * ((jx - 2 + h - 1) / h);
+        const long full = waves / kSlots, rest = waves % kSlots;
+        const double c = (h + 1.5) * (full * kShared + (rest == 0 ? 0.0 : (rest <= kSlots / kOcc ? kAlone : kShared)));
         if (c < cost) { cost = c; best = h; }
     }
     return best;
