@@ -205,6 +205,72 @@ def sum_sequential(xs):
     return t
 
 
+def _sides(kinds):
+    """Per (axis, side, field) kinds from four per-face entries (one kind, or seven)."""
+    return [k for face in kinds for k in (face if isinstance(face, (list, tuple)) else [face] * 7)]
+
+
+FRE, SPP, SPN, SMP, SMN, CNS, FRD, PER = range(8)
+WALL = [SPP, SPP, SPP, SPN, SPN, SPP, SPP]
+BOUNDS = {
+    "mirror and free": (FRE, FRE, WALL, FRE),
+    "mirrors": ([SPP, SPP, SPN, SPP, SPP, SPN, SPN], SMP, SMP, WALL),
+    "free and periodic": (FRE, SMP, PER, PER),
+    "periodic": (PER, PER, PER, PER),
+    # faces with another kind or a mixture: cfl_m, engine and fills one by one
+    "mixed": ([FRE, SPP, FRE, FRE, FRE, SPP, FRE], FRE, (SMP, SMP, SMP, SMN, SMP, SMN, SMP), FRE),
+    "constant and extrapolated": (FRE, FRD, PER, PER),
+}
+
+
+@pytest.mark.parametrize("bounds", list(BOUNDS))
+@pytest.mark.parametrize("nx,ny,margin", [(70, 33, 1), (65, 128, 2), (7, 9, 3), (4, 5, 1)])
+def test_mlw2d_resident_bounds(dev, oracle, bounds, nx, ny, margin):
+    """Resident runs with every face kind the fused kernel maps (and two that
+    it does not), signs per field, on stretched grids whose smallest
+    spacings lie in ghost cells; two calls of one run through MlwRun2D and
+    through Run, against cfl_m, mlw_m and the bd* of every field one after
+    the other.  The initial ghosts are not yet filled."""
+    from utrip_amd import cans
+    _print_case("mlw2d bounds", bounds, nx, ny, margin)
+    bc = _sides(BOUNDS[bounds])
+    ix, jx = nx + 2 * margin, ny + 2 * margin
+    s = smooth_state_2d(ix, jx, seed=ix + jx)
+    _, dx, dxm = stretched_grid(ix, seed=ix)
+    _, dy, dym = stretched_grid(jx, seed=jx + 7)
+    dx[0], dx[-1], dy[0], dy[-1] = 0.4 * dx.min(), 0.3 * dx.min(), 0.5 * dy.min(), 0.35 * dy.min()
+    f = {k: v.copy(order="F") for k, v in s.items()}
+    n, dts = 5, []
+    for _ in range(n):
+        dt, merr, _l = oracle.cfl_m_2d(0.3, 1e-10, 5.0 / 3.0, *[f[k] for k in F2[:6]], dx, dy)
+        assert merr == 0
+        oracle.mlw_m_2d(*[f[k] for k in F2], dt, 3.0, 5.0 / 3.0, dx, dxm, dy, dym)
+        for d in (0, 1):
+            for side in (0, 1):
+                for q, k in enumerate(F2):
+                    kind = bc[(2 * d + side) * 7 + q]
+                    if kind == PER:
+                        if side == 0:
+                            oracle.bnd_2d(d, PER, margin, margin, f[k])
+                    else:
+                        oracle.bnd_2d(d, kind, side, margin, f[k], 0.0, dxm if d == 0 else dym)
+        dts.append(dt)
+    gd = dict(dx=to_dev(dx, dev), dxm=to_dev(dxm, dev), dy=to_dev(dy, dev), dym=to_dev(dym, dev))
+    for kind in ("MlwRun2D", "Run"):
+        st = [to_dev(s[k], dev) for k in F2]
+        if kind == "Run":
+            run = cans.Run(2, cans.ENGINE_MLW, st, gd, 5.0 / 3.0, 0.3, qav=3.0, margin=margin, bc=bc)
+        else:
+            run = cans.MlwRun2D(st, gd["dx"], gd["dxm"], gd["dy"], gd["dym"], 3.0, 5.0 / 3.0, 0.3, margin=margin, bc=bc)
+        run.reset(dtmin=1e-10)
+        run.steps(2)
+        run.steps(n - 2)
+        cur, info = run.state()
+        assert info["nexec"] == n and info["dt"] == dts[-1], (kind, info, dts)
+        for k, t in zip(F2, cur):
+            assert_bitwise(to_host(t), f[k], f"{kind} {k}")
+
+
 @pytest.mark.parametrize("nx,ny", [(64, 61), (255, 250), (311, 401), (700, 130)])
 def test_mlw2d_resident_rows_per_wave(dev, oracle, nx, ny):
     """Resident periodic runs on grids whose strips take 1 to 5 rows per wave

@@ -460,9 +460,13 @@ int cans_run(int dim, int engine, int mixed, double *const *a, double *const *b,
     if (engine == CANS_ENGINE_MLWS && (dim == 1 || !bx1d))
         return abi_fail(CANS_ERR_ARG, "cans_run: mlw_m_s is 2D/3D and needs x, xm, y, ym (packed in bx1d)");
     if (engine < CANS_ENGINE_MLW || engine > CANS_ENGINE_MLWS) return abi_fail(CANS_ERR_ARG, "cans_run: engine %d", engine);
-    if (engine == CANS_ENGINE_MLW && dim == 2 && !bc)
-        return cans2d_mlw_run(a, b, clk, step0, nsteps, qav, gm, safety, dx, dxm, ix, dy, dym, jx, nullptr, margin,
-                              (double *)ws, events, stream);
+    if (engine == CANS_ENGINE_MLW && dim == 2) {   // no bc: the periodic box; one map a face: the same fused kernel
+        BndMap map;
+        const int nn[2] = {ix, jx};
+        if (!bc || (safety > 0.0 && bnd_map(bc, 2, 7, nn, margin, &map)))
+            return cans2d_mlw_run(a, b, clk, step0, nsteps, qav, gm, safety, dx, dxm, ix, dy, dym, jx, bc, margin,
+                                  (double *)ws, events, stream);
+    }
     if (!bc) return abi_fail(CANS_ERR_ARG, "cans_run: bc is NULL (only 2D MLW has the fused periodic path)");
     if (dim == 1) { jx = 1; kx = 1; }
     if (dim == 2) kx = 1;

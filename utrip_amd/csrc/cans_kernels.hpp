@@ -51,7 +51,7 @@ struct Mlw2dArgs {
     Clock *clk;        // non-null: dt and the run flag come from the clock
     int step;          // step index n for the clock
     int ix, jx;
-    int per_margin;    // > 0: also write the periodic ghost images (width)
+    int per_margin;    // > 0: also write the ghost images (width); a periodic box, or as launch_mlw2d's map says
     double safety;     // > 0 with clk: fused cfl_m of the new state
     int peek;          // 1: a clock kernel of this step already ran (read, do not advance)
     double *dt_log;    // non-null: dt_log[step] = the dt this step used
@@ -83,6 +83,49 @@ enum BndKind : int {
 };
 
 constexpr int kMaxBndFields = 16;
+
+// Faces whose ghost cells are copies of interior cells, the same cell for
+// every field and up to the sign: bdfre*, bdsp*, bdsm* (kept sign) and
+// bdper*.  bd*x, then bd*y, then bd*z then leave every ghost cell equal to
+// one interior cell, axis by axis through the face's index map, each field
+// times the product of its faces' signs.
+enum BndMapKind : int { BM_FRE = 0, BM_SP = 1, BM_SM = 2, BM_PER = 3 };
+struct BndMap {
+    int kind[3][2];        // per axis and side, a BndMapKind
+    unsigned neg[3][2];    // bit f: field f changes sign there (bdspn*)
+};
+// The map of a run's boundary list bc (per axis, side and field) on n[0..dim)
+// cells with ghost width m >= 1; false where a face mixes maps, has another
+// kind (bdsmn* writes an interior cell, bdcns*, bdfrd*, none), or reaches past the interior.
+inline bool bnd_map(const int *bc, int dim, int nf, const int *n, int m, BndMap *out) {
+    if (!bc || m < 1) return false;
+    for (int d = 0; d < dim; d++) {
+        for (int side = 0; side < 2; side++) {
+            const int *k = bc + (d * 2 + side) * nf;
+            int kind = -1;
+            unsigned neg = 0;
+            for (int f = 0; f < nf; f++) {
+                int c;
+                switch (k[f]) {
+                case BD_FRE: c = BM_FRE; break;
+                case BD_SPP: c = BM_SP; break;
+                case BD_SPN: c = BM_SP; neg |= 1u << f; break;
+                case BD_SMP: c = BM_SM; break;
+                case BD_PER: c = BM_PER; break;
+                default: return false;
+                }
+                if (kind >= 0 && c != kind) return false;
+                kind = c;
+            }
+            const int in = n[d] - 2 * m;   // interior cells
+            if (in < (kind == BM_FRE ? 1 : kind == BM_SM ? m + 1 : m)) return false;
+            out->kind[d][side] = kind;
+            out->neg[d][side] = neg;
+        }
+        if ((out->kind[d][0] == BM_PER) != (out->kind[d][1] == BM_PER)) return false;
+    }
+    return true;
+}
 struct BndArgs {
     double *q[kMaxBndFields];
     double q0[kMaxBndFields];
@@ -280,7 +323,7 @@ constexpr int kAdjAccSlot = kAdjStripes + 1;
 hipError_t launch_copy6(double *const *dst, double *const *src, size_t n, hipStream_t s);
 
 hipError_t launch_metric(const double *d, const double *dm, int n, Metric m, hipStream_t s);
-hipError_t launch_mlw2d(const Mlw2dArgs &a, hipStream_t s);
+hipError_t launch_mlw2d(const Mlw2dArgs &a, hipStream_t s, const BndMap *map = nullptr);
 hipError_t launch_mlw1d(const Mlw1dArgs &a, hipStream_t s);
 hipError_t launch_bnd(const BndArgs &a, hipStream_t s);
 // every field periodic on every face (margin m along each of the dim axes):

@@ -54,6 +54,54 @@ struct Prim {
     double ro, pr, vx, vy, bx, by;
 };
 
+// Where the ghost images of a cell lie: PerBox, the periodic box of the
+// plain resident run (the benchmark's; its code has no look-ups), or Faces, a
+// BndMap packed into two words: per face (axis * 2 + side) two bits of kinds
+// and eight of neg.
+struct PerBox {};
+struct Faces {
+    unsigned kinds, neg;
+    CANS_DEV int kind(int axis, int side) const { return (int)(kinds >> (4 * axis + 2 * side)) & 3; }
+    CANS_DEV unsigned sign(int axis, int side) const { return (neg >> (16 * axis + 8 * side)) & 127u; }
+    // the same words, opaque to the compiler: the rare rows and strips at an
+    // edge unpack them there instead of holding the pieces through the march
+    CANS_DEV Faces here() const {
+        Faces f = *this;
+        asm volatile("" : "+s"(f.kinds), "+s"(f.neg));
+        return f;
+    }
+};
+template <class M> constexpr bool kMapped = false;
+template <> constexpr bool kMapped<Faces> = true;
+
+// The ghost cells of one axis (n cells, width m) that are copies of cell i:
+// lo_n from lo_t up on the low side, hi_n from hi_t up on the high side.
+struct Images {
+    int lo_n, lo_t, hi_n, hi_t;
+    CANS_DEV int count() const { return lo_n + hi_n; }
+    CANS_DEV int at(int k) const { return k < lo_n ? lo_t + k : hi_t + k - lo_n; }
+};
+CANS_DEV Images images_of(const Faces &b, int axis, int i, int n, int m) {
+    Images r{0, 0, 0, 0};
+    const int lo = b.kind(axis, 0), hi = b.kind(axis, 1), e = n - m;
+    if (lo == BM_FRE) { r.lo_t = 1; r.lo_n = i == m + 1 ? m : 0; }                                     // bdfrex.f
+    else if (lo == BM_SP) { r.lo_t = 2 * m + 1 - i; r.lo_n = i >= m + 1 && i <= 2 * m; }               // bdsppx.f
+    else if (lo == BM_SM) { r.lo_t = 2 * m + 2 - i; r.lo_n = i >= m + 2 && i <= 2 * m + 1; }           // bdsmpx.f
+    else { r.lo_t = i - (n - 2 * m); r.lo_n = i >= n - 2 * m + 1 && i <= e; }                          // bdperx.f
+    if (hi == BM_FRE) { r.hi_t = e + 1; r.hi_n = i == e ? m : 0; }
+    else if (hi == BM_SP) { r.hi_t = 2 * e + 1 - i; r.hi_n = i >= e - m + 1 && i <= e; }
+    else if (hi == BM_SM) { r.hi_t = 2 * e - i; r.hi_n = i >= e - m && i <= e - 1; }
+    else { r.hi_t = i + (n - 2 * m); r.hi_n = i >= m + 1 && i <= 2 * m; }
+    return r;
+}
+// smallest of d at cell i and at its images
+CANS_DEV double images_min(const Faces &b, int axis, const double *d, int i, int n, int m) {
+    double g = d[i - 1];
+    const Images r = images_of(b, axis, i, n, m);
+    for (int k = 0; k < r.count(); k++) g = fminF(g, d[r.at(k) - 1]);
+    return g;
+}
+
 // Conserved variables and cell-centred fluxes of one cell (mlw_m.f:101-176).
 // x fluxes of the six equations: rx, eex, rxx, ryx, 0, -ez
 // y fluxes:                      ry, eey, rxy, ryy, ez, 0
@@ -102,7 +150,8 @@ struct ColCtx {
     double ux0, ux1;              // 0.5*dxm(i)/dx(i), 0.5*dxm(i-1)/dx(i)
     double qxs;                   // qav*dxm(i)
     double dxc;                   // dx(i)
-    double dxg;                   // min of dx(i) and dx of i's periodic x images
+    double dxg;                   // min of dx(i) and dx of i's x images
+    bool edge;                    // mapped: a column of the strip has x images (uniform)
 };
 
 // Row j (clamped to the grid, so every lane reads a real cell) of a field:
@@ -305,7 +354,8 @@ CANS_DEV double eq_xy(const RowCoef &r, double fE, double fC, double gN, double 
 // [m+1, jx-m], store and enter the CFL: the reference's bdperx/bdpery
 // overwrite what mlw_m computed in the ghost cells 2..m and ix-m+1..ix-1
 // with interior images.
-CANS_DEV void finish_row(const Mlw2dArgs &a, const YMet &y, const ColCtx &x, int j, const RowState &s,
+template <class M>
+CANS_DEV void finish_row(const Mlw2dArgs &a, const M &map, const YMet &y, const ColCtx &x, int j, const RowState &s,
                          bool do_cfl, double &dtmin_local) {
     const int mgj = a.per_margin;
     const bool out = x.out && (mgj == 0 || (j >= mgj + 1 && j <= a.jx - mgj));   // uniform in j
@@ -332,8 +382,12 @@ CANS_DEV void finish_row(const Mlw2dArgs &a, const YMet &y, const ColCtx &x, int
         // for bit: one division per cell and no per-image metric loads.
         const int mg = a.per_margin, jx = a.jx;
         double dyg = y.dy[j - 1];
-        if (mg > 0 && j >= jx - 2 * mg + 1) dyg = fminF(dyg, y.dy[j - (jx - 2 * mg) - 1]);
-        if (mg > 0 && j <= 2 * mg) dyg = fminF(dyg, y.dy[j + (jx - 2 * mg) - 1]);
+        if constexpr (kMapped<M>) {
+            if (j <= 2 * mg + 1 || j >= jx - 2 * mg) dyg = images_min(map.here(), 1, y.dy, j, jx, mg);
+        } else {
+            if (mg > 0 && j >= jx - 2 * mg + 1) dyg = fminF(dyg, y.dy[j - (jx - 2 * mg) - 1]);
+            if (mg > 0 && j <= 2 * mg) dyg = fminF(dyg, y.dy[j + (jx - 2 * mg) - 1]);
+        }
         const double dtq = a.safety * (fminF(x.dxg, dyg) / sq);
         dtmin_local = (out && dtq < dtmin_local) ? dtq : dtmin_local;
     }
@@ -349,10 +403,29 @@ CANS_DEV void finish_row(const Mlw2dArgs &a, const YMet &y, const ColCtx &x, int
         st(a.vy_o + rw, bo, vy); st(a.bx_o + rw, bo, bx); st(a.by_o + rw, bo, by);
         st(a.az_o + rw, bo, az);
         // In a periodic box also the ghost images: after bdperx then
-        // bdpery, ghost (gi,gj) holds interior (src_x(gi), src_y(gj)).
-        const int mg = a.per_margin;   // the host checks ix-2m >= m and jx-2m >= m
+        // bdpery, ghost (gi,gj) holds interior (src_x(gi), src_y(gj)); with a
+        // map likewise, each field times the signs of the faces.
+        const int mg = a.per_margin;   // the host checks ix-2m >= m and jx-2m >= m (bnd_map for a map)
         const int i = x.i;
-        if (mg > 0 && (i >= ix - 2 * mg + 1 || i <= 2 * mg || j >= jx - 2 * mg + 1 || j <= 2 * mg)) {
+        if constexpr (kMapped<M>) {
+            if (x.edge || j <= 2 * mg + 1 || j >= jx - 2 * mg) {   // uniform
+                const Faces map_ = map.here();
+                const Images xi = images_of(map_, 0, i, ix, mg), yj = images_of(map_, 1, j, jx, mg);
+                for (int b = -1; b < yj.count(); b++) {
+                    const int tj = b < 0 ? j : yj.at(b);
+                    const unsigned ny = b < 0 ? 0u : map_.sign(1, b < yj.lo_n ? 0 : 1);
+                    for (int c = b < 0 ? 0 : -1; c < xi.count(); c++) {
+                        const int t = c < 0 ? i : xi.at(c);
+                        const unsigned ng = ny ^ (c < 0 ? 0u : map_.sign(0, c < xi.lo_n ? 0 : 1));
+                        const size_t q = (size_t)(t - 1) + (size_t)ix * (size_t)(tj - 1);
+                        a.ro_o[q] = ng & 1u ? -ro : ro; a.pr_o[q] = ng & 2u ? -pr : pr;
+                        a.vx_o[q] = ng & 4u ? -vx : vx; a.vy_o[q] = ng & 8u ? -vy : vy;
+                        a.bx_o[q] = ng & 16u ? -bx : bx; a.by_o[q] = ng & 32u ? -by : by;
+                        a.az_o[q] = ng & 64u ? -az : az;
+                    }
+                }
+            }
+        } else if (mg > 0 && (i >= ix - 2 * mg + 1 || i <= 2 * mg || j >= jx - 2 * mg + 1 || j <= 2 * mg)) {
             int xi[3] = {i, 0, 0}, yj[3] = {j, 0, 0};
             int nxi = 1, nyj = 1;
             if (i >= ix - 2 * mg + 1) xi[nxi++] = i - (ix - 2 * mg);   // low ghost  <- high interior
@@ -374,8 +447,9 @@ CANS_DEV void finish_row(const Mlw2dArgs &a, const YMet &y, const ColCtx &x, int
 // One output row j: s holds the state entering row j, o receives the state
 // entering row j+1.  Everything but the stores runs on all 64 lanes (the
 // lane shifts need every lane's operands).
-CANS_DEV void row_step(const Mlw2dArgs &a, const YMet &y, const ColCtx &x, int j, double dt, bool do_cfl,
-                       const RowState &s, RowState &o, double &dtmin_local) {
+template <class M>
+CANS_DEV void row_step(const Mlw2dArgs &a, const M &map, const YMet &y, const ColCtx &x, int j, double dt,
+                       bool do_cfl, const RowState &s, RowState &o, double &dtmin_local) {
     j = __builtin_amdgcn_readfirstlane(j);   // wave-uniform: SGPR row bases and scalar loads
     const double gm = a.gm;
     // prefetch the row after next and the az of the next row
@@ -452,14 +526,15 @@ CANS_DEV void row_step(const Mlw2dArgs &a, const YMet &y, const ColCtx &x, int j
     o.ky[0] = C.roy; o.ky[1] = C.eey; o.ky[2] = C.rxy; o.ky[3] = C.ryy; o.ky[4] = C.ez;
     o.PS = PN;
 
-    finish_row(a, y, x, j, o, do_cfl, dtmin_local);
+    finish_row(a, map, y, x, j, o, do_cfl, dtmin_local);
 }
 
 // One wave's strip: columns 1+strip*COLS .. (lane 0 the west halo), output
 // rows jb = 2+rowb*H .. min(jb+H-1, jx-1), marched in y (prologue: the cells
 // of rows jb-1 and jb and the corner row jb-1).
-CANS_DEV void march_strip(const Mlw2dArgs &a, const YMet &y, int H, int strip, int rowb, double dt, bool do_cfl,
-                          double &dtmin_local) {
+template <class M>
+CANS_DEV void march_strip(const Mlw2dArgs &a, const M &map, const YMet &y, int H, int strip, int rowb, double dt,
+                          bool do_cfl, double &dtmin_local) {
     const int ix = a.ix, jx = a.jx;
     const int lane = threadIdx.x & (WAVE - 1);
     const int jb = 2 + rowb * H;
@@ -485,7 +560,11 @@ CANS_DEV void march_strip(const Mlw2dArgs &a, const YMet &y, int H, int strip, i
     x.qxs = a.qav * a.dxm[ic - 1];
     x.dxc = a.dx[ic - 1];
     x.dxg = x.dxc;
-    {
+    if constexpr (kMapped<M>) {
+        const int mg = a.per_margin;
+        x.edge = strip * COLS < 2 * mg + 1 || (strip + 1) * COLS + 1 >= ix - 2 * mg;
+        x.dxg = images_min(map, 0, a.dx, ic, ix, mg);
+    } else {
         const int mg = a.per_margin;
         if (mg > 0 && ic >= ix - 2 * mg + 1) x.dxg = fminF(x.dxg, a.dx[ic - (ix - 2 * mg) - 1]);
         if (mg > 0 && ic <= 2 * mg) x.dxg = fminF(x.dxg, a.dx[ic + (ix - 2 * mg) - 1]);
@@ -522,18 +601,18 @@ CANS_DEV void march_strip(const Mlw2dArgs &a, const YMet &y, int H, int strip, i
         if (q4 == 1) __builtin_amdgcn_s_setprio(2);
         else if (q4 == 2) __builtin_amdgcn_s_setprio(1);
         else if (q4 >= 3) __builtin_amdgcn_s_setprio(0);
-        row_step(a, y, x, j, dt, do_cfl, s0, s1, dtmin_local);
-        row_step(a, y, x, j + 1, dt, do_cfl, s1, s0, dtmin_local);
+        row_step(a, map, y, x, j, dt, do_cfl, s0, s1, dtmin_local);
+        row_step(a, map, y, x, j + 1, dt, do_cfl, s1, s0, dtmin_local);
     }
-    if (j <= je) row_step(a, y, x, j, dt, do_cfl, s0, s1, dtmin_local);
+    if (j <= je) row_step(a, map, y, x, j, dt, do_cfl, s0, s1, dtmin_local);
 }
 
 // The y metric arrays come as separate non-aliased arguments (the same
 // pointers as a.my, a.dym, a.dy) so that their per-row uniform loads go
 // through the scalar cache.
-template <int OCC>
+template <int OCC, class M>
 __global__ __launch_bounds__(WAVE * WPB) __attribute__((amdgpu_waves_per_eu(OCC))) void mlw2d_kernel(
-    Mlw2dArgs a, int H, const double *__restrict__ ydim, const double *__restrict__ ydi,
+    Mlw2dArgs a, M map, int H, const double *__restrict__ ydim, const double *__restrict__ ydi,
     const double *__restrict__ yu0, const double *__restrict__ yu1, const double *__restrict__ ydym,
     const double *__restrict__ ydy) {
     const YMet y{ydim, ydi, yu0, yu1, ydym, ydy};
@@ -557,7 +636,7 @@ __global__ __launch_bounds__(WAVE * WPB) __attribute__((amdgpu_waves_per_eu(OCC)
     const bool do_cfl = a.clk && a.safety > 0.0;
     double dtmin_local = kR4_1e20;
 
-    if (unit < nstrip * nrowb) march_strip(a, y, H, unit % nstrip, unit / nstrip, dt, do_cfl, dtmin_local);
+    if (unit < nstrip * nrowb) march_strip(a, map, y, H, unit % nstrip, unit / nstrip, dt, do_cfl, dtmin_local);
     if (do_cfl) block_min_to_global(dtmin_local, red, &a.clk->dtkey[(a.step + 1) % 3]);
 }
 
@@ -638,7 +717,7 @@ __global__ __launch_bounds__(BT) __attribute__((amdgpu_waves_per_eu(kOccBatch)))
             const Mlw2dArgs &a = b.runs[2 * k + (nexec & 1)];
             const YMet y{a.my.dim, a.my.di, a.my.u0, a.my.u1, a.dym, a.dy};
             double dmin = kR4_1e20;
-            for (int u = wv; u < nunit; u += NW) march_strip(a, y, H, u % nstrip, u / nstrip, dt, true, dmin);
+            for (int u = wv; u < nunit; u += NW) march_strip(a, PerBox{}, y, H, u % nstrip, u / nstrip, dt, true, dmin);
             nexec++;
             dt = block_min<BT>(dmin, red[par]);           // dt of the next step; also the step's barrier
             par ^= 1;
@@ -733,14 +812,25 @@ hipError_t launch_batch2d(const Batch2dArgs &b, int block_threads, int nblocks, 
     return hipGetLastError();
 }
 
-hipError_t launch_mlw2d(const Mlw2dArgs &a, hipStream_t s) {
+hipError_t launch_mlw2d(const Mlw2dArgs &a, hipStream_t s, const BndMap *map) {
     if (a.ix < 3 || a.jx < 3) return hipSuccess;
     const int h = pick_rows(a.ix, a.jx);
     const int nstrip = (a.ix - 2 + COLS - 1) / COLS;
     const int nrowb = (a.jx - 2 + h - 1) / h;
     const int nblocks = (nstrip * nrowb + WPB - 1) / WPB;
-    hipLaunchKernelGGL(mlw2d_kernel<kOcc>, dim3(nblocks), dim3(WAVE * WPB), 0, s, a, h, a.my.dim, a.my.di, a.my.u0,
-                       a.my.u1, a.dym, a.dy);
+    if (map) {
+        Faces f{0, 0};
+        for (int d = 0; d < 2; d++)
+            for (int side = 0; side < 2; side++) {
+                f.kinds |= (unsigned)map->kind[d][side] << (4 * d + 2 * side);
+                f.neg |= map->neg[d][side] << (16 * d + 8 * side);
+            }
+        hipLaunchKernelGGL((mlw2d_kernel<kOcc, Faces>), dim3(nblocks), dim3(WAVE * WPB), 0, s, a, f, h, a.my.dim,
+                           a.my.di, a.my.u0, a.my.u1, a.dym, a.dy);
+    } else {
+        hipLaunchKernelGGL((mlw2d_kernel<kOcc, PerBox>), dim3(nblocks), dim3(WAVE * WPB), 0, s, a, PerBox{}, h,
+                           a.my.dim, a.my.di, a.my.u0, a.my.u1, a.dym, a.dy);
+    }
     return hipGetLastError();
 }
 
