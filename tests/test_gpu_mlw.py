@@ -271,6 +271,77 @@ def test_mlw2d_resident_bounds(dev, oracle, bounds, nx, ny, margin):
             assert_bitwise(to_host(t), f[k], f"{kind} {k}")
 
 
+# cell counts on both sides of each buffer class of the one-launch 1D run
+# (coefficients and state in LDS, state in LDS, memory), of its block sizes
+# and of its longest tube; every face kind it maps, and two it does not
+@pytest.mark.parametrize("faces", [(FRE, FRE), ([SPP, SPP, SPN, SPP, SPN], FRE), (SMP, [SPP, SPP, SPN, SPN, SPP]),
+                                   (FRE, SMP), (PER, PER), ([SMP, SMP, SMN, SMP, SMP], FRE), (FRE, CNS)])
+@pytest.mark.parametrize("nx,margin", [(5, 1), (248, 1), (249, 3), (497, 2), (1260, 2), (1261, 2), (2028, 2), (2029, 2),
+                                       (4798, 1), (4799, 1)])
+def test_run_1d_bounds(dev, oracle, faces, nx, margin):
+    """Resident 1D MLW runs in three calls (1, 4 and 6 steps): the state, dt
+    and the buffer set of the step before, against cfl_m, mlw_m and the bd*
+    of every field one after the other; ghost spacings are the smallest."""
+    from utrip_amd import cans
+    _print_case("run 1d bounds", faces, nx, margin)
+    bc = [k for face in faces for k in (face if isinstance(face, list) else [face] * 5)]
+    ix = nx + 2 * margin
+    s = smooth_state_1d(ix, seed=ix)
+    _, dx, dxm = stretched_grid(ix, seed=ix)
+    dx[0], dx[-1] = 0.4 * dx.min(), 0.3 * dx.min()
+    dx[1], dx[-2] = 0.5 * dx[1:-1].min(), 0.6 * dx[1:-1].min()
+    f = {k: s[k].copy() for k in F1}
+    n, dts, prev = 11, [], None
+    for _ in range(n):
+        prev = {k: v.copy() for k, v in f.items()}
+        dt, merr, _i = oracle.cfl_m_1d(0.3, 1e-12, 5.0 / 3.0, s["bx"], *[f[k] for k in F1], dx)
+        assert merr == 0
+        oracle.mlw_m_1d(*[f[k] for k in F1], s["bx"], s["bxm"], dt, 3.0, 5.0 / 3.0, dx, dxm)
+        for side in (0, 1):
+            for q, k in enumerate(F1):
+                kind = bc[side * 5 + q]
+                if kind == PER:
+                    if side == 0:
+                        oracle.bnd_1d(PER, margin, margin, f[k])
+                else:
+                    oracle.bnd_1d(kind, side, margin, f[k], 0.0, dxm)
+        dts.append(dt)
+    gd = dict(dx=to_dev(dx, dev), dxm=to_dev(dxm, dev))
+
+    def run_of(**reset):
+        r = cans.Run(1, cans.ENGINE_MLW, [to_dev(s[k], dev) for k in F1], gd, 5.0 / 3.0, 0.3, qav=3.0, margin=margin,
+                     bc=bc, bx1d=to_dev(s["bx"], dev), bxm1d=to_dev(s["bxm"], dev))
+        r.reset(dtmin=1e-12, **reset)
+        for k in (1, 4, 6):
+            r.steps(k)
+        return r
+
+    run = run_of()
+    cur, info = run.state()
+    t = 0.0
+    for d in dts:
+        t = t + d
+    assert info == dict(t=t, ns=n, nexec=n, merr=0, dt=dts[-1])
+    other = run.a if cur is run.b else run.b
+    for k, q, r in zip(F1, cur, other):
+        assert_bitwise(to_host(q), f[k], k)
+        assert_bitwise(to_host(r), prev[k], "step before: " + k)
+    # stops on nstop and on tend, in the middle of a call and for good
+    info7 = run_of(nstop=7).state()[1]
+    assert info7["ns"] == info7["nexec"] == 7 and info7["dt"] == dts[6]
+    end = run_of(tend=info7["t"]).state()[1]
+    assert end["nexec"] == 7 and end["t"] == info7["t"]
+    r = cans.Run(1, cans.ENGINE_MLW, [to_dev(s[k], dev) for k in F1], gd, 5.0 / 3.0, 0.3, qav=3.0, margin=margin,
+                 bc=bc, bx1d=to_dev(s["bx"], dev), bxm1d=to_dev(s["bxm"], dev))
+    r.reset(dtmin=1.0)
+    r.steps(3)
+    cur, info = r.state()
+    assert info["merr"] == 9001 and info["nexec"] == 0 and info["ns"] == 1
+    inner = slice(margin + 1, ix - margin - 1)   # (single fills also run after the stop)
+    for k, q in zip(F1, cur):
+        assert_bitwise(to_host(q)[inner], s[k][inner], k)
+
+
 @pytest.mark.parametrize("nx,ny", [(64, 61), (255, 250), (311, 401), (700, 130)])
 def test_mlw2d_resident_rows_per_wave(dev, oracle, nx, ny):
     """Resident periodic runs on grids whose strips take 1 to 5 rows per wave

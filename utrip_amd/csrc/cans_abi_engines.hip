@@ -495,6 +495,24 @@ int cans_run(int dim, int engine, int mixed, double *const *a, double *const *b,
         if (dim >= 2) HIPCHK(launch_metric(dy, dym, jx, m[1], s));
         if (dim == 3) HIPCHK(launch_metric(dz, dzm, kx, m[2], s));
     }
+    // 1D MLW whose faces copy interior cells: all the call's steps in one launch
+    // (events bracket single steps, so a call with events takes them one by one)
+    BndMap map1;
+    if (engine == CANS_ENGINE_MLW && dim == 1 && !events && nsteps > 0 && safety > 0.0 && ix <= kRun1dMax &&
+        bnd_map(bc, 1, 5, n, margin, &map1)) {
+        Run1dArgs g{};
+        for (int f = 0; f < 5; f++) { g.a[f] = a[f]; g.b[f] = b[f]; }
+        g.bx = bx1d; g.bxm = bxm1d; g.dx = dx; g.dxm = dxm; g.di = m[0].di; g.dim = m[0].dim;
+        g.gm = gm; g.qav = qav; g.safety = safety; g.clk = c;
+        g.ix = ix; g.margin = margin;
+        for (int side = 0; side < 2; side++) { g.kind[side] = map1.kind[0][side]; g.neg[side] = map1.neg[0][side]; }
+        for (int st = 0; st < nsteps; st += kRun1dSteps) {   // launches of some 10 ms, others' work comes in between
+            g.step0 = step0 + st;
+            g.nsteps = nsteps - st < kRun1dSteps ? nsteps - st : kRun1dSteps;
+            HIPCHK(launch_run1d(g, s));
+        }
+        return 0;
+    }
     double *eng = cv.p;
     // In a periodic box (every field periodic on every face) the engine's
     // kernels carry cfl_m and the clock, so a step is the engine and the

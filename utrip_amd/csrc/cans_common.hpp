@@ -71,14 +71,35 @@ inline double dunkey_host(uint64_t k) {
     return d;
 }
 
-// Wavefront (64 lanes) min of a double; NaN never wins because the caller
-// only feeds values that passed `v < current`.
-CANS_DEV double wave_min(double v) {
-    for (int off = 32; off > 0; off >>= 1) {
-        double o = __shfl_xor(v, off, 64);
-        v = (o < v) ? o : v;
-    }
+// v with the lanes a DPP control moves replaced by their source lane's value
+// (the others keep their own).
+template <int CTRL, int ROWS>
+CANS_DEV double dpp_or_self(double v) {
+    const int lo = __double2loint(v), hi = __double2hiint(v);
+    return __hiloint2double(__builtin_amdgcn_update_dpp(hi, hi, CTRL, ROWS, 0xf, false),
+                            __builtin_amdgcn_update_dpp(lo, lo, CTRL, ROWS, 0xf, false));
+}
+CANS_DEV double read_lane(double v, int lane) {
+    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), lane),
+                            __builtin_amdgcn_readlane(__double2loint(v), lane));
+}
+// Lane 15 of each row of 16 lanes: the row's min (row_shr 1, 2, 4, 8).
+CANS_DEV double row_min15(double v) {
+    double o = dpp_or_self<0x111, 0xf>(v); v = (o < v) ? o : v;
+    o = dpp_or_self<0x112, 0xf>(v); v = (o < v) ? o : v;
+    o = dpp_or_self<0x114, 0xf>(v); v = (o < v) ? o : v;
+    o = dpp_or_self<0x118, 0xf>(v); v = (o < v) ? o : v;
     return v;
+}
+// Wavefront (64 lanes, all active) min of a double, uniform; NaN never wins
+// because the caller only feeds values that passed `v < current`.  By DPP
+// (rows, then row_bcast 15 and 31 into the next rows): the six LDS permutes
+// of a shuffle cost a step of a one-workgroup loop 0.3 us.
+CANS_DEV double wave_min(double v) {
+    v = row_min15(v);
+    double o = dpp_or_self<0x142, 0xa>(v); v = (o < v) ? o : v;
+    o = dpp_or_self<0x143, 0xc>(v); v = (o < v) ? o : v;
+    return read_lane(v, 63);
 }
 
 // Block min through LDS, then one atomic per block on the order-preserving

@@ -138,6 +138,24 @@ struct BndArgs {
     int ix, jx, kx;
 };
 
+// Steps step0 .. step0+nsteps-1 of one resident 1D MLW run in one launch
+// (cans_run1d.hip); its faces are those of a BndMap.
+struct Run1dArgs {
+    double *a[5], *b[5];                             // buffer sets: ro pr vx vy by
+    const double *bx, *bxm, *dx, *dxm, *di, *dim;
+    double gm, qav, safety;
+    Clock *clk;
+    int ix, margin, step0, nsteps;
+    int kind[2];
+    unsigned neg[2];
+};
+// Longest tube (cells, ghosts included) that runs so: beyond it, one CU's
+// issue costs more per step than a launch per routine across the chip (4000
+// cells 14.4 us a step against 17.1, 8000 cells 26.4 against 17.2).
+constexpr int kRun1dMax = 4800;
+constexpr int kRun1dSteps = 4096;   // steps a launch
+hipError_t launch_run1d(const Run1dArgs &a, hipStream_t s);
+
 struct CflArgs {
     const double *ro, *pr, *vx, *vy, *vz, *bx, *by, *bz;
     const double *dx, *dy, *dz;

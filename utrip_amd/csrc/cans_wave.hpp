@@ -48,10 +48,9 @@ CANS_DEV double block_min(double v, double *red) {
     v = wave_min(v);                       // the same value in every lane
     red[threadIdx.x >> 6] = v;             // all lanes store it: no divergent branch
     __syncthreads();
-    double m = red[0];
-#pragma unroll
-    for (int w = 1; w < NW; w++) m = (red[w] < m) ? red[w] : m;
-    return uni(m);
+    // a lane per wave's value, then the row min: no serial chain over NW
+    static_assert(NW <= 16 && (NW & (NW - 1)) == 0, "waves of a block");
+    return read_lane(row_min15(red[threadIdx.x & (NW - 1)]), 15);
 }
 
 // one term of the 1D cfl_m (cans1d/common/cfl_m.f:42-52: onero, ca2, cs2,
