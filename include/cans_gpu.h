@@ -479,8 +479,8 @@ int cans1d_batch_run_steps(int ntube, const long long *off, const int *ix, const
  * leaves the final state in state7, t, ns and merr (9001 if dt < dtmin).
  * block_threads in {64,...,512} with block_threads*blocks_per_cu <= 512.
  * ws: cans2d_batch_ws_bytes (tune = 1 adds room for cans2d_batch_tune's
- * copy of the state).  The call synchronises the stream once (to upload the
- * per-run argument table into ws), then launches asynchronously.  No single
+ * copy of the state).  The call reads the layout arrays back to check them,
+ * then launches asynchronously.  No single
  * counterpart in the reference, whose 2D driver runs one problem. */
 size_t cans2d_batch_ws_bytes(long long ncells, long long nx1d, long long ny1d, int nrun, int tune);
 int cans2d_batch_run(int nrun, const long long *off, const int *ix, const int *jx, const long long *offx,
@@ -504,8 +504,7 @@ int cans2d_batch_tune(int nrun, const long long *off, const int *ix, const int *
 /* cans2d_batch_run captured as an instantiated hipGraph (*graph; replay
  * with cans_graph_launch, free with cans_graph_destroy).  init7 (7 device
  * pointers, or NULL): copied into state7 at the start of every replay, so
- * replays repeat the same run.  The per-run argument table is uploaded into
- * ws before the capture; the graph reads it from there, so ws must not be
+ * replays repeat the same run.  The graph works in ws, which must not be
  * used by other calls while the graph is in use. */
 int cans2d_batch_graph(int nrun, const long long *off, const int *ix, const int *jx, const long long *offx,
                        const long long *offy, const int *order, double *const *state7, const double *dx,

@@ -302,12 +302,22 @@ int cans_graph_destroy(void *graph) {
 namespace {
 
 // workspace: the scratch state (7 fields), the x and y metric (4 arrays
-// each), the per-run argument table (2 per run), the queue counter, and
-// (tune) a copy of the state for the tuner's probes
-size_t b2_table_bytes(int nrun) { return (2 * (size_t)nrun * sizeof(Mlw2dArgs) + 255) & ~size_t(255); }
+// each), the queues, and (tune) a copy of the state for the tuner's probes
+// the queues of the shared runs: per group its counters and a ring of words
+// (a word of every run, and of every workgroup's late ticket, fits)
+unsigned b2_cap(int nrun) {
+    unsigned c = 8192;
+    while (c < (unsigned)nrun + 4096u) c *= 2;
+    return c;
+}
+size_t b2_ctl_bytes(int nrun) { return ((size_t)nrun * sizeof(Batch2dCtl) + 255) & ~size_t(255); }
+size_t b2_queue_bytes(int nrun) {
+    return 256 + kBatch2dGroups * (sizeof(Batch2dGroup) + (size_t)b2_cap(nrun) * sizeof(unsigned long long)) +
+           b2_ctl_bytes(nrun);
+}
 size_t b2_ws_bytes(long long ncells, long long nx1d, long long ny1d, int nrun, int tune) {
     return (7 * al((size_t)ncells) + 4 * al((size_t)nx1d) + 4 * al((size_t)ny1d)) * sizeof(double) +
-           b2_table_bytes(nrun) + 256 + (tune ? 7 * al((size_t)ncells) * sizeof(double) : 0);
+           b2_queue_bytes(nrun) + (tune ? 7 * al((size_t)ncells) * sizeof(double) : 0);
 }
 double *b2_tune_copy(void *ws, long long ncells, long long nx1d, long long ny1d, int nrun) {
     return (double *)((char *)ws + b2_ws_bytes(ncells, nx1d, ny1d, nrun, 0));
@@ -336,9 +346,8 @@ std::map<Tune2Key, std::pair<int, int>> &tune2_cache() {
     return m;
 }
 
-// Checks the layout on the host (the kernel trusts it), fills the launch
-// arguments for the state `state7` and uploads the per-run argument table
-// (synchronously: the host copy must outlive the transfer).
+// Checks the layout on the host (the kernel trusts it) and fills the launch
+// arguments for the state `state7`.
 int b2_prepare(const char *who, int nrun, const long long *off, const int *ix, const int *jx, const long long *offx,
                const long long *offy, const int *order, double *const *state7, const double *dx, const double *dxm,
                const double *dy, const double *dym, long long ncells, long long nx1d, long long ny1d, double gm,
@@ -392,36 +401,17 @@ int b2_prepare(const char *who, int nrun, const long long *off, const int *ix, c
         b.mx[q] = w + 7 * nc + q * n1x;
         b.my[q] = w + 7 * nc + 4 * n1x + q * n1y;
     }
-    Mlw2dArgs *table = reinterpret_cast<Mlw2dArgs *>(w + 7 * nc + 4 * n1x + 4 * n1y);
-    b.next = reinterpret_cast<unsigned *>(reinterpret_cast<char *>(table) + b2_table_bytes(nrun));
-    b.runs = table;
+    char *qp = reinterpret_cast<char *>(w + 7 * nc + 4 * n1x + 4 * n1y);
+    b.next = reinterpret_cast<unsigned *>(qp);
+    b.group = reinterpret_cast<Batch2dGroup *>(qp + 256);
+    b.ctl = reinterpret_cast<Batch2dCtl *>(qp + 256 + kBatch2dGroups * sizeof(Batch2dGroup));
+    b.ring = reinterpret_cast<unsigned long long *>(qp + 256 + kBatch2dGroups * sizeof(Batch2dGroup) + b2_ctl_bytes(nrun));
+    b.ngroup = kBatch2dGroups;
+    b.cap = b2_cap(nrun);
     b.dx = dx; b.dxm = dxm; b.dy = dy; b.dym = dym;
     b.gm = gm; b.qav = qav; b.safety = safety; b.dtmin = dtmin; b.tend = tend;
     b.nstop = nstop; b.margin = margin;
     b.t_out = t_out; b.ns_out = ns_out; b.merr_out = merr_out;
-    if (nrun == 0) return 0;
-    // the per-run arguments of the strip march, one per step parity
-    std::vector<Mlw2dArgs> h(2 * (size_t)nrun);
-    for (int k = 0; k < nrun; k++)
-        for (int par = 0; par < 2; par++) {
-            Mlw2dArgs &a = h[2 * (size_t)k + par];
-            a = Mlw2dArgs{};
-            double *const *cur = par ? b.g : b.f;
-            double *const *nxt = par ? b.f : b.g;
-            a.ro = cur[0] + o[k]; a.pr = cur[1] + o[k]; a.vx = cur[2] + o[k]; a.vy = cur[3] + o[k];
-            a.bx = cur[4] + o[k]; a.by = cur[5] + o[k]; a.az = cur[6] + o[k];
-            a.ro_o = nxt[0] + o[k]; a.pr_o = nxt[1] + o[k]; a.vx_o = nxt[2] + o[k]; a.vy_o = nxt[3] + o[k];
-            a.bx_o = nxt[4] + o[k]; a.by_o = nxt[5] + o[k]; a.az_o = nxt[6] + o[k];
-            a.dx = dx + ox[k]; a.dxm = dxm + ox[k]; a.dy = dy + oy[k]; a.dym = dym + oy[k];
-            a.mx = Metric{b.mx[0] + ox[k], b.mx[1] + ox[k], b.mx[2] + ox[k], b.mx[3] + ox[k]};
-            a.my = Metric{b.my[0] + oy[k], b.my[1] + oy[k], b.my[2] + oy[k], b.my[3] + oy[k]};
-            a.qav = qav; a.gm = gm; a.dt = 0.0; a.clk = nullptr; a.step = 0;
-            a.ix = nx[k]; a.jx = ny[k];
-            a.per_margin = margin; a.safety = safety; a.peek = 0; a.dt_log = nullptr;
-        }
-    // ordered after any earlier work on the stream that reads the table
-    HIPCHK(hipMemcpyAsync(table, h.data(), h.size() * sizeof(Mlw2dArgs), hipMemcpyHostToDevice, s));
-    HIPCHK(hipStreamSynchronize(s));
     return 0;
 }
 
@@ -540,7 +530,6 @@ int cans2d_batch_graph(int nrun, const long long *off, const int *ix, const int 
     hipStream_t s;
     HIPCHK(hipStreamCreateWithFlags(&s, hipStreamNonBlocking));
     Batch2dArgs b;
-    // the table is uploaded before the capture; replays read it from the workspace
     if (int e = b2_prepare("cans2d_batch_graph", nrun, off, ix, jx, offx, offy, order, state7, dx, dxm, dy, dym,
                            ncells, nx1d, ny1d, gm, qav, safety, dtmin, tend, nstop, margin, t_out, ns_out, merr_out,
                            ws, s, b)) {

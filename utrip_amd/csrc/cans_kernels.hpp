@@ -203,13 +203,29 @@ struct Batch2dArgs {
     double *g[7];                         // scratch set of the same size
     const double *dx, *dxm, *dy, *dym;    // packed grid arrays
     double *mx[4], *my[4];                // packed metric (di, dim, u0, u1), filled by the launch
-    const Mlw2dArgs *__restrict__ runs;   // per run k: runs[2k] reads f writes g, runs[2k+1] the reverse
     double gm, qav, safety, dtmin, tend;
     int nstop, margin;                    // margin: the periodic ghost width
     double *t_out;                        // device, per run
     int *ns_out, *merr_out;               // device, per run
-    unsigned *next;                       // queue counter (zeroed by the launch)
+    unsigned *next;                       // list counter (zeroed by the launch)
+    struct Batch2dGroup *group;           // ngroup queues (zeroed by the launch)
+    struct Batch2dCtl *ctl;               // per run
+    unsigned long long *ring;             // ngroup x cap queue words
+    int ngroup;
+    unsigned cap;                         // a power of two over the runs and workgroups that can be in a queue
 };
+// a group's queue counters, a cache line each
+struct Batch2dGroup {
+    unsigned head, pad0[31], tail, pad1[31], resv, pad2[31], active, pad3[31];
+};
+// a shared run's step: its dt, the loop's t, ns, the steps done, the cut into
+// units, and what the units of the step in progress have reduced
+struct Batch2dCtl {
+    unsigned long long minkey, dt_bits, t_bits;
+    unsigned done;
+    int ns, nexec, H, nstrip, nunit;
+};
+constexpr int kBatch2dGroups = 8;         // the XCDs
 hipError_t launch_batch2d(const Batch2dArgs &b, int block_threads, int nblocks, hipStream_t s);
 
 // mlw_m3 (cans{1,2}d/hdmlw/mlw_m3.f): 1D fields ro pr vx vy vz by bz (bx,

@@ -95,7 +95,8 @@ CANS_DEV Images images_of(const Faces &b, int axis, int i, int n, int m) {
     return r;
 }
 // smallest of d at cell i and at its images
-CANS_DEV double images_min(const Faces &b, int axis, const double *d, int i, int n, int m) {
+template <class P>
+CANS_DEV double images_min(const Faces &b, int axis, P d, int i, int n, int m) {
     double g = d[i - 1];
     const Images r = images_of(b, axis, i, n, m);
     for (int k = 0; k < r.count(); k++) g = fminF(g, d[r.at(k) - 1]);
@@ -136,10 +137,13 @@ struct RowState {
     double pro, pee, prx, pry, pbx, pby, paz;   // updated cell (i, j)
 };
 
-// Per-row (y) constants, read through non-aliased pointers.
-struct YMet {
-    const double *dim, *di, *u0, *u1, *dym, *dy;
+// Per-row (y) constants: non-aliased kernel arguments (const double *) in the
+// single-run kernel, constant address space in the batched one, so that the
+// uniform loads are scalar.
+template <class P> struct YMet {
+    P dim, di, u0, u1, dym, dy;
 };
+typedef const __attribute__((address_space(4))) double *KPtr;
 
 // Per-column constants of a strip.
 struct ColCtx {
@@ -354,8 +358,8 @@ CANS_DEV double eq_xy(const RowCoef &r, double fE, double fC, double gN, double 
 // [m+1, jx-m], store and enter the CFL: the reference's bdperx/bdpery
 // overwrite what mlw_m computed in the ghost cells 2..m and ix-m+1..ix-1
 // with interior images.
-template <class M>
-CANS_DEV void finish_row(const Mlw2dArgs &a, const M &map, const YMet &y, const ColCtx &x, int j, const RowState &s,
+template <class M, class P>
+CANS_DEV void finish_row(const Mlw2dArgs &a, const M &map, const YMet<P> &y, const ColCtx &x, int j, const RowState &s,
                          bool do_cfl, double &dtmin_local) {
     const int mgj = a.per_margin;
     const bool out = x.out && (mgj == 0 || (j >= mgj + 1 && j <= a.jx - mgj));   // uniform in j
@@ -447,8 +451,8 @@ CANS_DEV void finish_row(const Mlw2dArgs &a, const M &map, const YMet &y, const 
 // One output row j: s holds the state entering row j, o receives the state
 // entering row j+1.  Everything but the stores runs on all 64 lanes (the
 // lane shifts need every lane's operands).
-template <class M>
-CANS_DEV void row_step(const Mlw2dArgs &a, const M &map, const YMet &y, const ColCtx &x, int j, double dt,
+template <class M, class P>
+CANS_DEV void row_step(const Mlw2dArgs &a, const M &map, const YMet<P> &y, const ColCtx &x, int j, double dt,
                        bool do_cfl, const RowState &s, RowState &o, double &dtmin_local) {
     j = __builtin_amdgcn_readfirstlane(j);   // wave-uniform: SGPR row bases and scalar loads
     const double gm = a.gm;
@@ -532,8 +536,8 @@ CANS_DEV void row_step(const Mlw2dArgs &a, const M &map, const YMet &y, const Co
 // One wave's strip: columns 1+strip*COLS .. (lane 0 the west halo), output
 // rows jb = 2+rowb*H .. min(jb+H-1, jx-1), marched in y (prologue: the cells
 // of rows jb-1 and jb and the corner row jb-1).
-template <class M>
-CANS_DEV void march_strip(const Mlw2dArgs &a, const M &map, const YMet &y, int H, int strip, int rowb, double dt,
+template <class M, class P>
+CANS_DEV void march_strip(const Mlw2dArgs &a, const M &map, const YMet<P> &y, int H, int strip, int rowb, double dt,
                           bool do_cfl, double &dtmin_local) {
     const int ix = a.ix, jx = a.jx;
     const int lane = threadIdx.x & (WAVE - 1);
@@ -615,7 +619,7 @@ __global__ __launch_bounds__(WAVE * WPB) __attribute__((amdgpu_waves_per_eu(OCC)
     Mlw2dArgs a, M map, int H, const double *__restrict__ ydim, const double *__restrict__ ydi,
     const double *__restrict__ yu0, const double *__restrict__ yu1, const double *__restrict__ ydym,
     const double *__restrict__ ydy) {
-    const YMet y{ydim, ydi, yu0, yu1, ydym, ydy};
+    const YMet<const double *> y{ydim, ydi, yu0, yu1, ydym, ydy};
     __shared__ double red[WPB];
     const int ix = a.ix, jx = a.jx;
     const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -645,93 +649,298 @@ __global__ __launch_bounds__(WAVE * WPB) __attribute__((amdgpu_waves_per_eu(OCC)
 // (cans2d/md_mhdshktb/hdmlw/main.f:150-206 with bdperx/bdpery):
 //     ns=ns+1; cfl_m; stop on merr; t=t+dt; mlw_m; bdperx; bdpery;
 //     repeat while ns < nstop and t < tend
-// to its own end, in one persistent kernel.  A workgroup takes a run from a
-// queue and advances it to the end before taking the next; inside a run its
-// waves share the strips of each step (the register-marching strip of the
-// single-run kernel, with the ghost images and the next step's cfl term
-// fused), and a step ends with one workgroup barrier, the dt min-reduction.
-// Writes of one step are read by other waves of the same workgroup in the
-// next, after that barrier (one CU, one L1).
+// to its own end, in one persistent kernel.  A step's work is its strips'
+// units (march_strip: H rows of 62 columns, with the ghost images and the
+// next step's cfl term), a wave a unit.
+//
+// A workgroup takes runs from a list, costliest first.  A small run (under
+// kShareRounds rounds of units on the workgroup's waves) it advances by
+// itself, a step a turn; its only synchronisation is the workgroup's.  The
+// steps of a larger run are shared: whoever started the run, or finished the
+// last unit of its step, puts the next step into the queue of its group of
+// workgroups (those of one XCD, so that a run's state stays in one L2; runs
+// are dealt to the groups in turn), and workgroups take NW units at a time
+// from there, or from another group's when theirs has none, before anything
+// else.  One workgroup per run left the card to the longest runs: 192 runs of
+// 32..256 cells a side took 46.5 ms, the time of the costliest one on its CU.
+//
+// Nothing waits for a workgroup that may not be resident: a unit in a queue
+// is ready to run, units are taken only by running workgroups, and the one
+// that finishes a step's last unit queues the next.  A workgroup with
+// nothing to do polls until there is no shared run left (`active`), which
+// running workgroups bring about.  (The waiting inside a push is for an
+// earlier push of the group to be published, a few instructions of a running
+// wave.)
+//
+// Visibility: a wave waits for its stores (vmcnt 0) before the workgroup
+// barrier, wave 0 then adds its units to the step's `done` count with
+// agent-scope release; the last to add acquires, pushes with release, and who
+// takes units acquires before its waves load.
+enum { B2_UNITS, B2_OWN, B2_START, B2_IDLE, B2_EXIT };
+constexpr int kShareRounds = 3;
+constexpr int kShareRuns = 1 << 24;        // run numbers fit a queue word
+constexpr int kShareUnits = 1 << 15;       // units of a step fit, with room for late tickets
 
-// rows per strip for a run of jx rows and nstrip strips on NW waves: the
-// fewest rounds of units, each unit's prologue counted as 1.5 rows
-CANS_DEV int batch2d_rows(int jx, int nstrip, int NW) {
-    int best = 8;
+CANS_DEV unsigned long long ald(const unsigned long long *p) {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+CANS_DEV unsigned ald(const unsigned *p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+CANS_DEV int ald(const int *p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+template <class T> CANS_DEV void ast(T *p, T v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+// one lane's atomic add, its old value in every lane
+CANS_DEV unsigned add1(unsigned *p, unsigned v) {
+    unsigned r = 0;
+    if ((threadIdx.x & 63) == 0) r = __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return (unsigned)uni((int)r);
+}
+CANS_DEV unsigned long long add1(unsigned long long *p, unsigned long long v) {
+    unsigned long long r = 0;
+    if ((threadIdx.x & 63) == 0) r = __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return (unsigned long long)uni((long long)r);
+}
+
+// The rows per unit and the units of a run of ix x jx cells: the fewest
+// rounds of NW units, a unit's prologue counted as 1.5 rows and its share of
+// the round's synchronisation as 2.5.
+struct B2Cut {
+    int H, nstrip, nunit;
+};
+CANS_DEV B2Cut batch2d_cut(int ix, int jx, int NW) {
+    B2Cut c{8, (ix - 2 + COLS - 1) / COLS, 0};
     double cost = 1e300;
-    for (int h = 4; h <= 48; h++) {
-        const int units = nstrip * ((jx - 2 + h - 1) / h);
-        const double c = (double)((units + NW - 1) / NW) * (h + 1.5);
-        if (c < cost) { cost = c; best = h; }
+    for (int h = 4; h <= 16; h++) {
+        const int units = c.nstrip * ((jx - 2 + h - 1) / h);
+        const double q = (double)((units + NW - 1) / NW) * (h + 4.0);
+        if (q < cost) { cost = q; c.H = h; }
     }
-    return best;
+    for (;; c.H *= 2) {
+        c.nunit = c.nstrip * ((jx - 2 + c.H - 1) / c.H);
+        if (c.nunit <= kShareUnits || c.H >= jx) break;
+    }
+    return c;
+}
+
+// The queue of a group: words (run, units, next ticket) in a ring; [head,
+// tail) are published, resv counts the reserved.
+CANS_DEV void b2_push(const Batch2dArgs &b, int grp, int k, int nunit) {
+    Batch2dGroup &g = b.group[grp];
+    const unsigned idx = add1(&g.resv, 1u);
+    if ((threadIdx.x & 63) == 0)
+        __hip_atomic_store(&b.ring[(size_t)grp * b.cap + (idx & (b.cap - 1))],
+                           ((unsigned long long)k << 40) | ((unsigned long long)nunit << 24), __ATOMIC_RELEASE,
+                           __HIP_MEMORY_SCOPE_AGENT);
+    while ((unsigned)uni((int)ald(&g.tail)) != idx) __builtin_amdgcn_s_sleep(1);
+    if ((threadIdx.x & 63) == 0)
+        __hip_atomic_store(&g.tail, idx + 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
+}
+// What wave 0 found for its workgroup to do: units of its own group's queue,
+// else of another's; a step of the workgroup's own run; the next run.
+struct B2Do {
+    int op, k, unit, grp;
+};
+CANS_DEV B2Do b2_next(const Batch2dArgs &b, int grp, int NW, bool own) {
+    const int lane = threadIdx.x & 63, ng = b.ngroup;
+    for (;;) {
+        unsigned h = 0, t = 0;
+        if (lane < ng) { h = ald(&b.group[lane].head); t = ald(&b.group[lane].tail); }
+        const unsigned full = (unsigned)__ballot((int)(t - h) > 0);
+        if (full == 0) break;
+        const unsigned turned = (full >> grp) | (full << (ng - grp));   // bit 0: the own group
+        const int g = (grp + __builtin_ctz(turned)) % ng;
+        const unsigned hg = (unsigned)__builtin_amdgcn_readlane((int)h, g);
+        const unsigned long long w = add1(&b.ring[(size_t)g * b.cap + (hg & (b.cap - 1))], (unsigned long long)NW);
+        const int u = (int)(w & 0xffffffull), n = (int)((w >> 24) & 0xffffull);
+        if (u < n) {
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+            return B2Do{B2_UNITS, (int)(w >> 40), u, g};
+        }
+        if (lane == 0) {   // every unit of the head is taken: the next word
+            unsigned want = hg;
+            __hip_atomic_compare_exchange_strong(&b.group[g].head, &want, hg + 1u, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                                 __HIP_MEMORY_SCOPE_AGENT);
+        }
+    }
+    if (own) return B2Do{B2_OWN, 0, 0, 0};
+    unsigned *active = &b.group[0].active;   // shared runs, and workgroups that may be starting one
+    if (uni((int)ald(b.next)) < b.nrun) {
+        add1(active, 1u);
+        const int q = (int)add1(b.next, 1u);
+        if (q < b.nrun) return B2Do{B2_START, b.order ? uni(b.order[q]) : q, 0, q % ng};
+        add1(active, ~0u);
+    }
+    return B2Do{uni((int)ald(active)) > 0 ? B2_IDLE : B2_EXIT, 0, 0, 0};
+}
+
+// The march's arguments of run k for step parity par (0 reads the state and
+// writes the scratch, 1 the reverse).
+CANS_DEV Mlw2dArgs b2_args(const Batch2dArgs &b, int k, int par) {
+    const long long o = uni(b.off[k]), ox = uni(b.offx[k]), oy = uni(b.offy[k]);
+    double *in[7], *out[7];
+#pragma unroll
+    for (int q = 0; q < 7; q++) {
+        in[q] = (par ? b.g[q] : b.f[q]) + o;
+        out[q] = (par ? b.f[q] : b.g[q]) + o;
+    }
+    Mlw2dArgs a;
+    a.ro = in[0]; a.pr = in[1]; a.vx = in[2]; a.vy = in[3]; a.bx = in[4]; a.by = in[5]; a.az = in[6];
+    a.ro_o = out[0]; a.pr_o = out[1]; a.vx_o = out[2]; a.vy_o = out[3]; a.bx_o = out[4]; a.by_o = out[5];
+    a.az_o = out[6];
+    a.dx = b.dx + ox; a.dxm = b.dxm + ox; a.dy = b.dy + oy; a.dym = b.dym + oy;
+    a.mx = Metric{b.mx[0] + ox, b.mx[1] + ox, b.mx[2] + ox, b.mx[3] + ox};
+    a.my = Metric{b.my[0] + oy, b.my[1] + oy, b.my[2] + oy, b.my[3] + oy};
+    a.qav = b.qav; a.gm = b.gm; a.dt = 0.0; a.clk = nullptr; a.step = 0;
+    a.ix = uni(b.ix[k]); a.jx = uni(b.jx[k]);
+    a.per_margin = b.margin; a.safety = b.safety; a.peek = 0; a.dt_log = nullptr;
+    return a;
 }
 
 template <int BT>
 __global__ __launch_bounds__(BT) __attribute__((amdgpu_waves_per_eu(kOccBatch))) void batch2d_kernel(Batch2dArgs b) {
     constexpr int NW = BT / 64;
     __shared__ double red[2][NW];
-    __shared__ int run_s;
+    // the work in hand: a run's step and the units of it, and what came of it
+    __shared__ struct { int op, k, grp, u0, u1, nexec, H, nstrip, nunit, end, ns, merr; double dt, t; } c;
+    __shared__ struct { int k, ns, nexec, H, nstrip, nunit; double dt, t; } own;   // the workgroup's own run (k >= 0)
     const int wv = uni((int)(threadIdx.x >> 6));
+    const int grp = (int)(blockIdx.x % (unsigned)b.ngroup);
+    int par = 0;
+    if (wv == 0) own.k = -1;
     for (;;) {
-        // queue pop by wave 0 under a uniform branch (lane 0 adds 1)
         if (wv == 0) {
-            const unsigned got = atomicAdd(b.next, threadIdx.x == 0 ? 1u : 0u);
-            run_s = uni((int)got);
+            const bool have = uni(own.k) >= 0;
+            const B2Do d = b2_next(b, grp, NW, have);
+            c.op = d.op; c.k = d.k; c.grp = d.grp; c.end = 0;
+            if (d.op == B2_UNITS) {
+                const Batch2dCtl &r = b.ctl[d.k];
+                const int n = uni(ald(&r.nunit));
+                c.nexec = uni(ald(&r.nexec)); c.H = uni(ald(&r.H)); c.nstrip = uni(ald(&r.nstrip)); c.nunit = n;
+                c.dt = __longlong_as_double(uni((long long)ald(&r.dt_bits)));
+                c.u0 = d.unit; c.u1 = min(d.unit + NW, n);
+            } else if (d.op == B2_OWN) {
+                c.k = own.k; c.nexec = own.nexec; c.H = own.H; c.nstrip = own.nstrip; c.nunit = own.nunit;
+                c.dt = own.dt; c.u0 = 0; c.u1 = own.nunit;
+            }
         }
         __syncthreads();
-        const int kq = uni(run_s);
-        __syncthreads();
-        if (kq >= b.nrun) break;
-        const int k = b.order ? uni(b.order[kq]) : kq;
-        const long long o = uni(b.off[k]);
-        // step parity p reads set p and writes the other: runs[2k+p]
-        const Mlw2dArgs &a0 = b.runs[2 * k];
-        const int ix = uni(a0.ix), jx = uni(a0.jx);
-        const size_t ncell = (size_t)ix * (size_t)jx;
-        // cfl_m of the initial state over every cell (cans2d/common/cfl_m.f:44-62)
-        double m = kR4_1e20;
-        for (size_t p = threadIdx.x; p < ncell; p += BT) {
-            const int i = (int)(p % (size_t)ix) + 1, j = (int)(p / (size_t)ix) + 1;
-            const size_t q = (size_t)o + p;
-            const double ro = b.f[0][q], pr = b.f[1][q], vx = b.f[2][q], vy = b.f[3][q], bx = b.f[4][q],
-                         by = b.f[5][q];
-            const double b2 = bx * bx + by * by;
-            const double ca2 = b2 * pi4i / ro;
-            const double cs2 = b.gm * pr / ro;
-            const double v2 = vx * vx + vy * vy;
-            const double dtq = b.safety * (fminF(a0.dx[i - 1], a0.dy[j - 1]) / __builtin_sqrt(v2 + cs2 + ca2));
-            if (dtq < m) m = dtq;
-        }
-        int par = 0;
-        double dt = block_min<BT>(m, red[par]);
-        par ^= 1;
-        int ns = 0, merr = 0, nexec = 0;
-        double t = 0.0;
-        const int nstrip = (ix - 2 + COLS - 1) / COLS;
-        const int H = batch2d_rows(jx, nstrip, NW);
-        const int nunit = nstrip * ((jx - 2 + H - 1) / H);
-        for (;;) {
-            ns = ns + 1;
-            if (dt < b.dtmin) { merr = 9001; break; }     // cfl_m.f: merr=9001, main.f stops
-            t = t + dt;
-            const Mlw2dArgs &a = b.runs[2 * k + (nexec & 1)];
-            const YMet y{a.my.dim, a.my.di, a.my.u0, a.my.u1, a.dym, a.dy};
-            double dmin = kR4_1e20;
-            for (int u = wv; u < nunit; u += NW) march_strip(a, PerBox{}, y, H, u % nstrip, u / nstrip, dt, true, dmin);
-            nexec++;
-            dt = block_min<BT>(dmin, red[par]);           // dt of the next step; also the step's barrier
+        const int op = uni(c.op), k = uni(c.k);
+        if (op == B2_EXIT) break;
+        if (op == B2_IDLE) {
+            __builtin_amdgcn_s_sleep(16);
+        } else if (op == B2_START) {
+            const long long o = uni(b.off[k]), ox = uni(b.offx[k]), oy = uni(b.offy[k]);
+            const int ix = uni(b.ix[k]), jx = uni(b.jx[k]);
+            const size_t ncell = (size_t)ix * (size_t)jx;
+            // cfl_m of the initial state over every cell (cans2d/common/cfl_m.f:44-62)
+            double m = kR4_1e20;
+            for (size_t p = threadIdx.x; p < ncell; p += BT) {
+                const int i = (int)(p % (size_t)ix) + 1, j = (int)(p / (size_t)ix) + 1;
+                const size_t q = (size_t)o + p;
+                const double ro = b.f[0][q], pr = b.f[1][q], vx = b.f[2][q], vy = b.f[3][q], bx = b.f[4][q],
+                             by = b.f[5][q];
+                const double b2 = bx * bx + by * by;
+                const double ca2 = b2 * pi4i / ro;
+                const double cs2 = b.gm * pr / ro;
+                const double v2 = vx * vx + vy * vy;
+                const double dtq = b.safety * (fminF(b.dx[ox + i - 1], b.dy[oy + j - 1]) / __builtin_sqrt(v2 + cs2 + ca2));
+                if (dtq < m) m = dtq;
+            }
+            const double dt = block_min<BT>(m, red[par]);
             par ^= 1;
-            if (!(ns < b.nstop && t < b.tend)) break;
+            if (wv == 0) {
+                const B2Cut cut = batch2d_cut(ix, jx, NW);
+                const bool bad = dt < b.dtmin;                 // cfl_m.f: merr=9001, main.f stops
+                const bool share = !bad && cut.nunit > (kShareRounds - 1) * NW && b.nrun < kShareRuns &&
+                                   cut.nunit <= kShareUnits;
+                if (share) {
+                    if (threadIdx.x == 0) {
+                        Batch2dCtl &r = b.ctl[k];
+                        ast(&r.done, 0u);
+                        ast(&r.minkey, (unsigned long long)dkey(kR4_1e20));
+                        ast(&r.dt_bits, (unsigned long long)__double_as_longlong(dt));
+                        ast(&r.t_bits, (unsigned long long)__double_as_longlong(0.0 + dt));
+                        ast(&r.ns, 1); ast(&r.nexec, 0); ast(&r.H, cut.H); ast(&r.nstrip, cut.nstrip);
+                        ast(&r.nunit, cut.nunit);
+                    }
+                    b2_push(b, uni(c.grp), k, cut.nunit);
+                } else {
+                    add1(&b.group[0].active, ~0u);
+                    if (bad) {
+                        c.end = 1; c.nexec = 0; c.ns = 1; c.merr = 9001; c.t = 0.0;
+                    } else {
+                        own.k = k; own.ns = 1; own.nexec = 0; own.dt = dt; own.t = 0.0 + dt;
+                        own.H = cut.H; own.nstrip = cut.nstrip; own.nunit = cut.nunit;
+                    }
+                }
+            }
+        } else {   // a step of the own run, or units of a shared run's step
+            {
+                const int nstrip = uni(c.nstrip), u1 = uni(c.u1), H = uni(c.H);
+                const double dt = uni(c.dt);
+                const Mlw2dArgs a = b2_args(b, k, uni(c.nexec) & 1);
+                const YMet<KPtr> y{(KPtr)a.my.dim, (KPtr)a.my.di, (KPtr)a.my.u0, (KPtr)a.my.u1, (KPtr)a.dym, (KPtr)a.dy};
+                double dmin = kR4_1e20;
+                for (int u = uni(c.u0) + wv; u < u1; u += NW)
+                    march_strip(a, PerBox{}, y, H, u % nstrip, u / nstrip, dt, true, dmin);
+                red[par][wv] = wave_min(dmin);
+            }
+            __builtin_amdgcn_s_waitcnt(0x0f70);   // this wave's stores have reached L2 (vmcnt 0)
+            __syncthreads();                      // (the own run's step ends here)
+            if (wv == 0) {
+                const double m = read_lane(row_min15(red[par][threadIdx.x & (NW - 1)]), 15);
+                Batch2dCtl &r = b.ctl[k];
+                const bool mine = op == B2_OWN;
+                const int u0 = uni(c.u0), u1 = uni(c.u1), nunit = uni(c.nunit), nexec = uni(c.nexec) + 1;
+                const unsigned cnt = (unsigned)(u1 - u0);
+                unsigned d = 0;
+                if (!mine && threadIdx.x == 0) {
+                    atomicMin(&r.minkey, (unsigned long long)dkey(m));
+                    d = __hip_atomic_fetch_add(&r.done, cnt, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
+                }
+                if ((unsigned)uni((int)d) + cnt == (unsigned)nunit) {   // the step's last units: its end and the next
+                    const double dt = mine ? m : dunkey((unsigned long long)uni((long long)ald(&r.minkey)));
+                    double t = mine ? own.t : __longlong_as_double(uni((long long)ald(&r.t_bits)));
+                    int ns = uni(mine ? own.ns : ald(&r.ns));
+                    const bool more = ns < b.nstop && uni(t) < b.tend;
+                    if (more) ns++;
+                    const bool bad = more && uni(dt) < b.dtmin;
+                    if (more && !bad) {
+                        t = t + dt;
+                        if (mine) {
+                            own.ns = ns; own.nexec = nexec; own.dt = dt; own.t = t;
+                        } else {
+                            if (threadIdx.x == 0) {
+                                ast(&r.done, 0u);
+                                ast(&r.minkey, (unsigned long long)dkey(kR4_1e20));
+                                ast(&r.dt_bits, (unsigned long long)__double_as_longlong(dt));
+                                ast(&r.t_bits, (unsigned long long)__double_as_longlong(t));
+                                ast(&r.ns, ns); ast(&r.nexec, nexec);
+                            }
+                            b2_push(b, uni(c.grp), k, nunit);
+                        }
+                    } else {
+                        c.end = 1; c.nexec = nexec; c.ns = ns; c.merr = bad ? 9001 : 0; c.t = t;
+                        if (mine) own.k = -1;
+                        else add1(&b.group[0].active, ~0u);
+                    }
+                }
+            }
+            par ^= 1;
         }
-        if (nexec & 1) {   // the last state is in the scratch set: copy back
-            for (size_t p = threadIdx.x; p < ncell; p += BT)
+        __syncthreads();
+        if (uni(c.end)) {
+            if (uni(c.nexec) & 1) {   // the last state is in the scratch set: copy back
+                const long long o = uni(b.off[k]);
+                const size_t ncell = (size_t)uni(b.ix[k]) * (size_t)uni(b.jx[k]);
+                for (size_t p = threadIdx.x; p < ncell; p += BT)
 #pragma unroll
-                for (int q = 0; q < 7; q++) b.f[q][(size_t)o + p] = b.g[q][(size_t)o + p];
-        }
-        if (wv == 0) {   // uniform branch; the lanes store identical values
-            b.t_out[k] = t;
-            b.ns_out[k] = ns;
-            b.merr_out[k] = merr;
+                    for (int q = 0; q < 7; q++) b.f[q][(size_t)o + p] = b.g[q][(size_t)o + p];
+            }
+            if (wv == 0) {   // uniform branch; the lanes store identical values
+                b.t_out[k] = c.t;
+                b.ns_out[k] = c.ns;
+                b.merr_out[k] = c.merr;
+            }
+            __syncthreads();   // every wave has read c before wave 0 writes it again
         }
     }
 }
@@ -740,7 +949,13 @@ __global__ __launch_bounds__(BT) __attribute__((amdgpu_waves_per_eu(kOccBatch)))
 // kernel) and the queue counter; block r fills run r
 __global__ void batch2d_prep(Batch2dArgs b) {
     const int r = blockIdx.x;
-    if (r == 0 && threadIdx.x == 0) *b.next = 0u;
+    if (r == 0) {
+        if (threadIdx.x == 0) *b.next = 0u;
+        if ((int)threadIdx.x < b.ngroup) {
+            Batch2dGroup &g = b.group[threadIdx.x];
+            g.head = g.tail = g.resv = g.active = 0u;
+        }
+    }
     if (r >= b.nrun) return;
     for (int axis = 0; axis < 2; axis++) {
         const long long o = axis ? b.offy[r] : b.offx[r];
