@@ -87,6 +87,64 @@ def test_batch2d_many_uneven_runs(dev, oracle):
     check_batch(oracle, list(zip(nx.tolist(), ny.tolist(), ps.tolist())), 1, tend=0.1, nstop=40, shape=(256, 2))
 
 
+@pytest.mark.parametrize("shape", [(512, 1), (128, 4)])
+def test_batch2d_shared_runs_on_two_streams(dev, oracle, shape):
+    """Runs whose steps are shared between workgroups (several rounds of
+    units, ragged last ones) beside small ones: two batches at once on two
+    streams, one of them stopping a run on dtmin, every run checked."""
+    from utrip_amd import cans
+    print("CASE batch2d shared runs, two streams", shape, flush=True)
+    specs = [(190, 170, 1.0), (64, 301, 3.0), (255, 40, 0.3), (20, 21, 1.0), (125, 126, 5.0)]
+    batches = []
+    for m, part in ((1, specs), (2, specs[1:])):
+        runs = []
+        for nx, ny, ps in part:
+            r, pp = make_run(nx, ny, m, ps)
+            runs.append(r)
+        s = torch.cuda.Stream()
+        with torch.cuda.stream(s):
+            b = cans.Batch2D(runs, pp["gm"], pp["qav"], pp["safety"], m, dtmin=3.586e-3 if m == 2 else 1e-10)
+        batches.append((b, runs, pp, m, s))
+    torch.cuda.synchronize()
+    for b, *_, s in batches:
+        with torch.cuda.stream(s):
+            b.run(tend=0.06, nstop=14, block_threads=shape[0], blocks_per_cu=shape[1])
+    torch.cuda.synchronize()
+    stopped = 0
+    for b, runs, pp, m, _s in batches:
+        t, ns, merr = b.t.cpu().numpy(), b.ns.cpu().numpy(), b.merr.cpu().numpy()
+        for k, r in enumerate(runs):
+            want = 0
+            if m == 2:   # the first step whose dt is under dtmin, if any
+                f, tr, nsr, want = oracle_to_dtmin(oracle, r, pp, m, 0.06, 14, 3.586e-3)
+                stopped += want == 9001
+            else:
+                f, tr, nsr = oracle_run(oracle, r, pp, m, 0.06, 14)
+            got = b.run_fields(k)
+            for q in F2:
+                assert_bitwise(got[q], f[q], f"margin {m} run {k} {q}")
+            assert t[k] == tr and ns[k] == nsr and merr[k] == want, (m, k, t[k], tr, ns[k], nsr)
+    assert stopped
+
+
+def oracle_to_dtmin(oracle, r, pp, m, tend, nstop, dtmin):
+    """oracle_run with a dtmin: the state, t, ns and merr where it stops."""
+    f = {k: r[k].copy(order="F") for k in F2}
+    t, ns = 0.0, 0
+    while True:
+        ns += 1
+        dt, merr, _ = oracle.cfl_m_2d(pp["safety"], dtmin, pp["gm"], *[f[k] for k in F2[:6]], r["dx"], r["dy"])
+        if merr:
+            return f, t, ns, merr
+        t = t + dt
+        oracle.mlw_m_2d(*[f[k] for k in F2], dt, pp["qav"], pp["gm"], r["dx"], r["dxm"], r["dy"], r["dym"])
+        for d in (0, 1):
+            for k in F2:
+                oracle.bnd_2d(d, 7, m, m, f[k])
+        if not (ns < nstop and t < tend):
+            return f, t, ns, 0
+
+
 def test_batch2d_second_run_restarts_from_state(dev, oracle):
     """A second run() starts every run's loop again (t = 0, ns = 0) from the
     state the first left, reusing the workspace and its queue counter; it

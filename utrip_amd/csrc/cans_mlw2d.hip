@@ -677,7 +677,11 @@ __global__ __launch_bounds__(WAVE * WPB) __attribute__((amdgpu_waves_per_eu(OCC)
 // agent-scope release; the last to add acquires, pushes with release, and who
 // takes units acquires before its waves load.
 enum { B2_UNITS, B2_OWN, B2_START, B2_IDLE, B2_EXIT };
-constexpr int kShareRounds = 3;
+// A run is shared from this many rounds of its workgroup's waves: at one round
+// the queue costs more than it spreads (1000 runs of 16..64 cells a side 3.0
+// against 1.1 ms), from two on it pays (192 runs of 32..256: 8.6 ms at two,
+// 10.9 at three, 15.9 at six; 1024 such runs 37 ms, 71.3 unshared).
+constexpr int kShareRounds = 2;
 constexpr int kShareRuns = 1 << 24;        // run numbers fit a queue word
 constexpr int kShareUnits = 1 << 15;       // units of a step fit, with room for late tickets
 
@@ -708,7 +712,7 @@ struct B2Cut {
 CANS_DEV B2Cut batch2d_cut(int ix, int jx, int NW) {
     B2Cut c{8, (ix - 2 + COLS - 1) / COLS, 0};
     double cost = 1e300;
-    for (int h = 4; h <= 16; h++) {
+    for (int h = 4; h <= 20; h++) {
         const int units = c.nstrip * ((jx - 2 + h - 1) / h);
         const double q = (double)((units + NW - 1) / NW) * (h + 4.0);
         if (q < cost) { cost = q; c.H = h; }
