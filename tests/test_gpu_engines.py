@@ -148,6 +148,28 @@ def test_bnd3d_kinds(dev, oracle, kind):
                 assert_bitwise(to_host(t), r, f"3d dir {d} kind {kind} side {mbnd} margin {margin}")
 
 
+@pytest.mark.parametrize("shape,margins", [((4, 5), (2, 2)), ((6, 4), (1, 3)), ((7, 9), (3, 4)), ((5, 3), (0, 1))])
+def test_bnd_short_lines(dev, oracle, shape, margins):
+    """Fills whose lines are about as short as their margins (a periodic one
+    then copies ghosts it has filled), uneven periodic margins, and none."""
+    from utrip_amd import cans
+    case("bnd short lines", shape, margins)
+    rng = np.random.default_rng(3)
+    for d in (0, 1):
+        n = shape[d]
+        dm = np.abs(rng.standard_normal(n)) + 0.1
+        for kind in range(8):
+            for mbnd, mg in ([margins, margins[::-1]] if kind == 7 else [(s, m) for s in (0, 1) for m in margins]):
+                if (mbnd + mg > n) if kind == 7 else (2 * mg + 1 > n):   # refused
+                    continue
+                q = np.asfortranarray(rng.standard_normal(shape))
+                r = q.copy(order="F")
+                oracle.bnd_2d(d, kind, mbnd, mg, r, 0.37, dm)
+                t = to_dev(q, dev)
+                cans.bnd_2d(d, kind, mbnd, mg, t, 0.37, to_dev(dm, dev))
+                assert_bitwise(to_host(t), r, f"dir {d} kind {kind} mbnd {mbnd} margin {mg}")
+
+
 # ------------------------------------------------------------------ resident runs
 def oracle_loop(oracle, dim, engine, fields, grid, pp, nsteps, bc_kind, margin, bx=None, bxm=None, mu=1.0):
     """The reference main loop on the CPU: cfl_m, engine, bnd (all fields,
@@ -184,7 +206,7 @@ def oracle_loop(oracle, dim, engine, fields, grid, pp, nsteps, bc_kind, margin, 
                 oracle.roe_m_3d(*[f[k] for k in F3], dt, pp["gm"], grid["dx"], grid["dy"], grid["dz"])
         else:
             oracle.hlld_engine(*[f[k] for k in F3], pp["gm"], mu, dt, grid["dx"], grid["dy"], grid["dz"], (1, 1, 1))
-        for d in range(dim):
+        for d in range(dim if bc_kind >= 0 else 0):   # (-1: no fills)
             dm = grid[("dxm", "dym", "dzm")[d]]
             for k in names:
                 if bc_kind == 7:
@@ -272,6 +294,57 @@ def test_run_periodic_fill_shapes(dev, oracle, shape, margin):
     assert info["nexec"] == 6 and info["merr"] == 0 and info["dt"] == dts[-1]
     for k in {1: F1, 2: F2, 3: F3}[dim]:
         assert_bitwise(got[k], ref[k], k)
+
+
+@pytest.mark.parametrize("engine,shape,margin", [("mlw", (13, 12, 11), 1), ("mlw", (11, 13, 14), 2), ("roe", (13, 12, 14), 3),
+                                                 ("hlld", (12, 13, 13), 3), ("roe", (20, 17), 3), ("roe", (30,), 3)])
+@pytest.mark.parametrize("faces", ["mirror", "mixed"])
+def test_run_mapped_fill(dev, oracle, engine, shape, margin, faces):
+    """Runs whose ghost fill is the one pass over free, mirror (both kinds,
+    signs per field) and periodic faces, and ("mixed") runs that fill face
+    by face because one face has two kinds, against the bd* of every field
+    one after the other."""
+    case("run mapped fill", engine, shape, margin, faces)
+    from utrip_amd import cans
+    dim = len(shape)
+    names = {1: F1, 2: F2, 3: F3}[dim]
+    nf = len(names)
+    FRE, SPP, SPN, SMP, PER = 0, 1, 2, 3, 7
+    wall = [SPN if k[0] in "vb" and k[1] == "xyz"[0] else SPP for k in names]
+    bc = ([SPP] * (nf - 1) + [FRE] if faces == "mixed" else wall) + [FRE] * nf
+    if dim >= 2:
+        bc += [SMP] * nf + [SPP] * nf
+    if dim == 3:
+        bc += [PER] * (2 * nf)
+    n = [s + 2 * margin for s in shape]
+    f = {1: smooth_state_1d, 2: smooth_state_2d, 3: smooth_state_3d}[dim](*n, seed=7)
+    g = {}
+    for ax, m in zip("xyz", n):
+        _, g["d" + ax], g["d" + ax + "m"] = stretched_grid(m, seed=m)
+    ref = {k: f[k].copy(order="F") for k in names}
+    pp = dict(gm=5.0 / 3.0, safety=0.3, qav=3.0, dtmin=1e-12)
+    for _ in range(4):
+        # one step of the loop without its fills, then the fills face by face
+        ref, dts = oracle_loop(oracle, dim, engine, ref, g, pp, 1, -1, margin, f.get("bx"), f.get("bxm"))
+        for d in range(dim):
+            for side in (0, 1):
+                for q, k in enumerate(names):
+                    kind = bc[(2 * d + side) * nf + q]
+                    if kind == PER and side == 1:
+                        continue
+                    args = (kind, margin if kind == PER else side, margin, ref[k])
+                    oracle.bnd_1d(*args) if dim == 1 else (oracle.bnd_2d if dim == 2 else oracle.bnd_3d)(d, *args)
+    st = [to_dev(f[k], dev) for k in names]
+    run = cans.Run(dim, {"mlw": cans.ENGINE_MLW, "roe": cans.ENGINE_ROE, "hlld": cans.ENGINE_HLLD}[engine], st,
+                   {k: to_dev(v, dev) for k, v in g.items()}, pp["gm"], pp["safety"], qav=pp["qav"], margin=margin, bc=bc,
+                   bx1d=to_dev(f["bx"], dev) if dim == 1 else None, bxm1d=to_dev(f["bxm"], dev) if dim == 1 else None)
+    run.reset(dtmin=pp["dtmin"])
+    run.steps(1)
+    run.steps(3)
+    cur, info = run.state()
+    assert info["nexec"] == 4 and info["dt"] == dts[-1]
+    for k, q in zip(names, cur):
+        assert_bitwise(to_host(q), ref[k], k)
 
 
 @pytest.mark.parametrize("n,nsteps", [(40, 12), (724, 4)])

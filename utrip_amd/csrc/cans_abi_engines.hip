@@ -99,25 +99,17 @@ static int roe_dropin(int dim, bool mixed, double *const *prim, double *az, cons
     hipStream_t s = (hipStream_t)stream;
     const size_t N = (size_t)ix * jx * kx;
     void *w = nullptr;
-    if (int rc = abi_scratch((engine_doubles(dim, CANS_ENGINE_ROE, N) + 9 * al(N)) * sizeof(double), &w, s)) return rc;
+    if (int rc = abi_scratch(engine_doubles(dim, CANS_ENGINE_ROE, N) * sizeof(double), &w, s)) return rc;
     Carver c{(double *)w};
     RoeArgs r{};
-    for (int q = 0; q < 8; q++) r.prim[q] = prim[q];
+    // in place: once the half step is made, a cell's primitives and Az are read
+    // only by the thread that updates the cell, before it writes them
+    for (int q = 0; q < 8; q++) { r.prim[q] = prim[q]; r.out[q] = prim[q]; }
     roe_scratch(r, c, N, dim, comp3);
-    double *outbuf[8];
-    for (int q = 0; q < 8; q++) { outbuf[q] = c.take(N); r.out[q] = prim[q] ? outbuf[q] : nullptr; }
-    double *azo = c.take(N);
-    r.az = az; r.out_az = dim == 2 ? azo : nullptr;
+    r.az = az; r.out_az = dim == 2 ? az : nullptr;
     r.bx = bx; r.bxm = bxm; r.dx = dx; r.dy = dy; r.dz = dz;
     r.gm = gm; r.dt = dt; r.clk = nullptr; r.ix = ix; r.jx = jx; r.kx = kx;
     HIPCHK(launch_roe(r, dim, mixed, s, comp3));
-    double *dst[9];
-    const double *src[9];
-    int nf = 0;
-    for (int q = 0; q < 8; q++)
-        if (prim[q]) { dst[nf] = prim[q]; src[nf] = outbuf[q]; nf++; }
-    if (dim == 2) { dst[nf] = az; src[nf] = azo; nf++; }
-    HIPCHK(launch_copy_interior(dst, src, nf, ix, jx, kx, 3, s));
     return 0;
 }
 
@@ -495,17 +487,18 @@ int cans_run(int dim, int engine, int mixed, double *const *a, double *const *b,
         if (dim >= 2) HIPCHK(launch_metric(dy, dym, jx, m[1], s));
         if (dim == 3) HIPCHK(launch_metric(dz, dzm, kx, m[2], s));
     }
-    // 1D MLW whose faces copy interior cells: all the call's steps in one launch
-    // (events bracket single steps, so a call with events takes them one by one)
-    BndMap map1;
-    if (engine == CANS_ENGINE_MLW && dim == 1 && !events && nsteps > 0 && safety > 0.0 && ix <= kRun1dMax &&
-        bnd_map(bc, 1, 5, n, margin, &map1)) {
+    // the ghost cells are copies of interior cells, one map a face
+    BndMap map;
+    const bool mapped = bnd_map(bc, dim, nf, n, margin, &map);
+    // 1D MLW so: all the call's steps in one launch (events bracket single
+    // steps, so a call with events takes them one by one)
+    if (engine == CANS_ENGINE_MLW && dim == 1 && mapped && !events && nsteps > 0 && safety > 0.0 && ix <= kRun1dMax) {
         Run1dArgs g{};
         for (int f = 0; f < 5; f++) { g.a[f] = a[f]; g.b[f] = b[f]; }
         g.bx = bx1d; g.bxm = bxm1d; g.dx = dx; g.dxm = dxm; g.di = m[0].di; g.dim = m[0].dim;
         g.gm = gm; g.qav = qav; g.safety = safety; g.clk = c;
         g.ix = ix; g.margin = margin;
-        for (int side = 0; side < 2; side++) { g.kind[side] = map1.kind[0][side]; g.neg[side] = map1.neg[0][side]; }
+        for (int side = 0; side < 2; side++) { g.kind[side] = map.kind[0][side]; g.neg[side] = map.neg[0][side]; }
         for (int st = 0; st < nsteps; st += kRun1dSteps) {   // launches of some 10 ms, others' work comes in between
             g.step0 = step0 + st;
             g.nsteps = nsteps - st < kRun1dSteps ? nsteps - st : kRun1dSteps;
@@ -526,11 +519,9 @@ int cans_run(int dim, int engine, int mixed, double *const *a, double *const *b,
     //    own cfl_m and the next kernel advances the clock, after the first
     //    step of a call (whose ghost cells need not be images yet), which
     //    keeps the cfl pass and the clock kernel.
-    // (allper: every field periodic on every face; the ghost fill is then one
-    // pass, launch_bnd_periodic)
-    bool allper = margin >= 1 && bc != nullptr;
-    for (int k = 0; allper && k < 2 * dim * nf; k++) allper = bc[k] == BD_PER;
-    for (int d = 0; allper && d < dim; d++) allper = n[d] - 2 * margin >= margin;
+    // (mapped: the ghost fill is one pass, launch_bnd_map.  allper: all periodic)
+    bool allper = mapped;
+    for (int d = 0; allper && d < dim; d++) allper = map.kind[d][0] == BM_PER;   // (both sides or neither)
     const bool perio = allper && safety > 0.0;
     const bool per3 = perio && dim == 3 &&
                       ((engine == CANS_ENGINE_MLW && mlw3d_path() != 0) ||
@@ -668,8 +659,8 @@ int cans_run(int dim, int engine, int mixed, double *const *a, double *const *b,
         }
         if (events) HIPCHK(hipEventRecord((hipEvent_t)events[2 * e + 1], s));
         // bnd: x faces, then y, then z; each face: periodic fields both sides
-        if (allper) {
-            HIPCHK(launch_bnd_periodic(out, nf, ix, jx, kx, dim, margin, s));
+        if (mapped) {
+            HIPCHK(launch_bnd_map(out, nf, ix, jx, kx, dim, margin, map, s));
             continue;
         }
         for (int dir = 0; dir < dim; dir++) {

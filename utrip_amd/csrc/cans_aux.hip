@@ -28,127 +28,157 @@ __global__ void metric_kernel(const double *d, const double *dm, int n, Metric m
 }
 
 // ---------------------------------------------------------------- boundary
-// One thread per (field, line).  A line runs along `dir` through the array;
-// the fill is the 1D index map of cans1d/bc/*.f applied to that line, which
-// is what the 2D/3D routines do for every transverse index (including the
-// transverse ghosts, cans2d/bc/bdperx.f:31-44).
-__global__ void bnd_kernel(BndArgs a) {
-    const int n = a.dir == 0 ? a.ix : (a.dir == 1 ? a.jx : a.kx);
-    const long nlines = (long)a.ix * a.jx * a.kx / n;
-    const long gid = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    const int f = (int)(gid / nlines);
-    const long l = gid - (long)f * nlines;
-    if (f >= a.nf) return;
+// A line runs along `dir` through the array; the fill is the 1D index map of
+// cans1d/bc/*.f applied to that line, which is what the 2D/3D routines do for
+// every transverse index (including the transverse ghosts,
+// cans2d/bc/bdperx.f:31-44).  One thread per field, line and distance i from
+// the face (1..w, w the wider margin): its one or two ghost cells do not
+// depend on the others', except for bdfrd's running extrapolation and for a
+// periodic line too short for its margins, whose copies read ghosts filled
+// before them: there the thread of i = 1 fills the line in order.  Neighbour
+// threads run along memory: i first for x faces, the line otherwise.  I: the
+// index type, 32 bits where the faces fit (64-bit divisions were most of the
+// kernel).
+template <class I>
+struct BndLines {
+    I total, minor;          // threads a field; the extent of their faster index (i on x faces, else the line)
+    int ifast, n;            // 1: i is the faster index; cells of a line
+    I fast;                  // line l = slow * fast + fl lies at fl * sfast + slow * sslow
+    long sfast, sslow, stride;
+};
+template <class I>
+__global__ void bnd_kernel(BndArgs a, BndLines<I> g) {
+    const int f = (int)blockIdx.y;
+    const I r = (I)blockIdx.x * (I)blockDim.x + (I)threadIdx.x;
+    if (r >= g.total) return;
+    const I hi = r / g.minor, lo = r - hi * g.minor;
+    const I l = g.ifast ? hi : lo;
+    const int i = 1 + (int)(g.ifast ? lo : hi);
+    const int n = g.n;
     const int kind = a.kind[f];
     if (kind < 0) return;
-    // base offset and stride of the line
-    long base, stride;
-    if (a.dir == 0) { base = l * a.ix; stride = 1; }
-    else if (a.dir == 1) { const long i = l % a.ix, k = l / a.ix; base = i + k * (long)a.ix * a.jx; stride = a.ix; }
-    else { base = l; stride = (long)a.ix * a.jx; }
-    double *q = a.q[f] + base;
+    const I slow = l / g.fast;
+    const long stride = g.stride;
+    double *q = a.q[f] + ((long)(l - slow * g.fast) * g.sfast + (long)slow * g.sslow);
 #define Q(idx) q[(long)((idx) - 1) * stride]
     const int margin = a.margin;
     if (kind == BD_PER) {   // bdperx.f:31-40
         const int margin0 = a.mbnd, margin1 = a.margin;
         const int ibnd0 = 1 + margin0, ibnd1 = n - margin1;
-        for (int i = 1; i <= margin0; i++) Q(ibnd0 - i) = Q(ibnd1 + 1 - i);
-        for (int i = 1; i <= margin1; i++) Q(ibnd1 + i) = Q(ibnd0 - 1 + i);
+        const int in = n - margin0 - margin1;
+        if (in >= margin0 && in >= margin1) {
+            if (i <= margin0) Q(ibnd0 - i) = Q(ibnd1 + 1 - i);
+            if (i <= margin1) Q(ibnd1 + i) = Q(ibnd0 - 1 + i);
+        } else if (i == 1) {
+            for (int k = 1; k <= margin0; k++) Q(ibnd0 - k) = Q(ibnd1 + 1 - k);
+            for (int k = 1; k <= margin1; k++) Q(ibnd1 + k) = Q(ibnd0 - 1 + k);
+        }
         return;
     }
-    if (a.mbnd == 0) {
-        const int ibnd = 1 + margin;
-        double dqq = 0.0;
-        if (kind == BD_FRD) dqq = (Q(ibnd + 1) - Q(ibnd)) / a.dm[ibnd - 1];   // bdfrdx.f
-        for (int i = 1; i <= margin; i++) {
-            switch (kind) {
-            case BD_FRE: Q(ibnd - i) = Q(ibnd); break;            // bdfrex.f
-            case BD_SPP: Q(ibnd - i) = Q(ibnd - 1 + i); break;    // bdsppx.f
-            case BD_SPN: Q(ibnd - i) = -Q(ibnd - 1 + i); break;   // bdspnx.f
-            case BD_SMP: Q(ibnd - i) = Q(ibnd + i); break;        // bdsmpx.f
-            case BD_SMN: Q(ibnd - i) = -Q(ibnd + i); break;       // bdsmnx.f
-            case BD_CNS: Q(ibnd - i) = a.q0[f]; break;            // bdcnsx.f
-            case BD_FRD: Q(ibnd - i) = Q(ibnd - i + 1) - dqq * a.dm[ibnd - i - 1]; break;
-            default: break;
-            }
+    if (i > margin && !(kind == BD_SMN && i == 1)) return;
+    const int ibnd = a.mbnd == 0 ? 1 + margin : n - margin;
+    const int o = a.mbnd == 0 ? -1 : 1;          // outwards
+    switch (i <= margin ? kind : -1) {
+    case BD_FRE: Q(ibnd + o * i) = Q(ibnd); break;                // bdfrex.f
+    case BD_SPP: Q(ibnd + o * i) = Q(ibnd + o * (1 - i)); break;  // bdsppx.f
+    case BD_SPN: Q(ibnd + o * i) = -Q(ibnd + o * (1 - i)); break; // bdspnx.f
+    case BD_SMP: Q(ibnd + o * i) = Q(ibnd - o * i); break;        // bdsmpx.f
+    case BD_SMN: Q(ibnd + o * i) = -Q(ibnd - o * i); break;       // bdsmnx.f
+    case BD_CNS: Q(ibnd + o * i) = a.q0[f]; break;                // bdcnsx.f
+    case BD_FRD:                                                  // bdfrdx.f
+        if (i == 1 && a.mbnd == 0) {
+            const double dqq = (Q(ibnd + 1) - Q(ibnd)) / a.dm[ibnd - 1];
+            for (int k = 1; k <= margin; k++) Q(ibnd - k) = Q(ibnd - k + 1) - dqq * a.dm[ibnd - k - 1];
+        } else if (i == 1) {
+            const double dqq = (Q(ibnd) - Q(ibnd - 1)) / a.dm[ibnd - 2];
+            for (int k = 1; k <= margin; k++) Q(ibnd + k) = Q(ibnd + k - 1) + dqq * a.dm[ibnd + k - 2];
         }
-        if (kind == BD_SMN) Q(ibnd) = 0.0;
-    } else {
-        const int ibnd = n - margin;
-        double dqq = 0.0;
-        if (kind == BD_FRD) dqq = (Q(ibnd) - Q(ibnd - 1)) / a.dm[ibnd - 2];
-        for (int i = 1; i <= margin; i++) {
-            switch (kind) {
-            case BD_FRE: Q(ibnd + i) = Q(ibnd); break;
-            case BD_SPP: Q(ibnd + i) = Q(ibnd + 1 - i); break;
-            case BD_SPN: Q(ibnd + i) = -Q(ibnd + 1 - i); break;
-            case BD_SMP: Q(ibnd + i) = Q(ibnd - i); break;
-            case BD_SMN: Q(ibnd + i) = -Q(ibnd - i); break;
-            case BD_CNS: Q(ibnd + i) = a.q0[f]; break;
-            case BD_FRD: Q(ibnd + i) = Q(ibnd + i - 1) + dqq * a.dm[ibnd + i - 2]; break;
-            default: break;
-            }
-        }
-        if (kind == BD_SMN) Q(ibnd) = 0.0;
+        break;
+    default: break;
     }
+    if (kind == BD_SMN && i == 1) Q(ibnd) = 0.0;
 #undef Q
 }
 
-// Every field periodic on every face of a 1D/2D/3D box, all directions in
-// one pass.  bdperx, then bdpery, then bdperz (each over every transverse
-// index, the ghosts included) leave each ghost cell equal to the interior
-// cell at its images along every axis, i -> i +- (n - 2m) for a ghost index
-// (n - 2m >= m: one shift reaches the interior): each ghost cell is copied
-// from that cell directly, the same values.  Sources are interior cells,
-// which the pass never writes.  Wave units: (row with a ghost j or k, 64
-// columns) copy the whole row with lanes along x; then 64 (row, ghost
-// column) items of the rows whose j and k are interior.
-struct PerFill {
+// The faces of a BndMap, all directions in one pass.  bd*x, then bd*y, then
+// bd*z (each over every transverse index, the ghosts included) leave each
+// ghost cell equal to the interior cell at its images along every axis, times
+// the faces' signs: each ghost cell is copied from that cell directly, the
+// same values.  Sources are interior cells, which the pass never writes.
+// Wave units: (row with a ghost j or k, 64 columns) copy the whole row with
+// lanes along x; then 64 (row, ghost column) items of the rows whose j and k
+// are interior.  Periodic boxes: 3D step -0.6 to -1.1 % against three fills;
+// an open cylindrical run of 160x64x128 takes one launch instead of five.
+struct MapFill {
     double *q[kMaxBndFields];
-    int nf, ix, jx, kx, mx, my, mz;
+    int ix, jx, kx, mx, my, mz;
     long long na, nb;   // units of the two kinds
+    BndMap map;
 };
-CANS_DEV int per_img(int i, int n, int m) { return i <= m ? i + (n - 2 * m) : (i > n - m ? i - (n - 2 * m) : i); }
+// the interior index whose value index i takes along an axis
+CANS_DEV int map_img(const BndMap &b, int axis, int i, int n, int m, unsigned &neg) {
+    const int side = i <= m ? 0 : (i > n - m ? 1 : -1);
+    if (side < 0) return i;
+    neg ^= b.neg[axis][side];
+    const int e = side == 0 ? m + 1 : n - m, d = side == 0 ? e - i : i - e;   // e: first interior cell, d >= 1 outwards
+    const int in = side == 0 ? 1 : -1;
+    switch (b.kind[axis][side]) {
+    case BM_FRE: return e;
+    case BM_SP: return e + in * (d - 1);
+    case BM_SM: return e + in * d;
+    default: return side == 0 ? i + (n - 2 * m) : i - (n - 2 * m);
+    }
+}
 
-__global__ __launch_bounds__(256) void per_fill_kernel(PerFill a) {
+// I: the unit index type, 32 bits where the units and items fit.  NF: the
+// fields, all loaded before the first is stored (one after the other, a cell
+// waited for memory NF times).
+template <class I, int NF>
+__global__ __launch_bounds__(256) void map_fill_kernel(MapFill a) {
     const int ix = a.ix, jx = a.jx, kx = a.kx, mx = a.mx, my = a.my, mz = a.mz;
-    const long long nchunk = (ix + 63) / 64;
+    const I nchunk = (I)((ix + 63) / 64), na = (I)a.na, nu = (I)(a.na + a.nb);
     const int lane = threadIdx.x & 63;
-    const long long nw = (long long)gridDim.x * (blockDim.x >> 6);
-    for (long long u = uni((long long)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6)); u < a.na + a.nb; u += nw) {
+    const I nw = (I)gridDim.x * (I)(blockDim.x >> 6);
+    for (I u = uni((I)blockIdx.x * (I)(blockDim.x >> 6) + (I)(threadIdx.x >> 6)); u < nu; u += nw) {
         int i, j, k;
         bool on;
-        if (u < a.na) {
-            const long long g = u / nchunk;
+        if (u < na) {
+            const I g = u / nchunk;
             const int c = (int)(u - g * nchunk);
-            const long long gz = 2LL * mz * jx;   // rows of the ghost z planes
+            const I gz = 2 * (I)mz * (I)jx;       // rows of the ghost z planes
             if (g < gz) {
-                const int pk = (int)(g / jx);
-                j = (int)(g - (long long)pk * jx) + 1;
+                const int pk = (int)(g / (I)jx);
+                j = (int)(g - (I)pk * (I)jx) + 1;
                 k = pk < mz ? pk + 1 : kx - 2 * mz + pk + 1;
             } else {                               // interior planes: their ghost y rows
-                const long long h = g - gz;
-                const int pj = (int)(h % (2 * my));
-                k = mz + 1 + (int)(h / (2 * my));
+                const I h = g - gz, r = h / (I)(2 * my);
+                const int pj = (int)(h - r * (I)(2 * my));
+                k = mz + 1 + (int)r;
                 j = pj < my ? pj + 1 : jx - 2 * my + pj + 1;
             }
             i = c * 64 + lane + 1;
             on = i <= ix;
         } else {
-            const long long v = (u - a.na) * 64 + lane;
-            const long long nrow = (long long)(jx - 2 * my) * (kx - 2 * mz);
-            on = v < nrow * 2 * mx;
-            const int col = (int)(v % (2 * mx));
-            const long long r = v / (2 * mx);
-            j = my + 1 + (int)(r % (jx - 2 * my));
-            k = mz + 1 + (int)(r / (jx - 2 * my));
+            const I v = (u - na) * 64 + (I)lane;
+            const I nrow = (I)(jx - 2 * my) * (I)(kx - 2 * mz);
+            on = v < nrow * (I)(2 * mx);
+            const I r = v / (I)(2 * mx), p = r / (I)(jx - 2 * my);
+            const int col = (int)(v - r * (I)(2 * mx));
+            j = my + 1 + (int)(r - p * (I)(jx - 2 * my));
+            k = mz + 1 + (int)p;
             i = col < mx ? col + 1 : ix - 2 * mx + col + 1;
         }
         if (on) {
             const size_t dst = (size_t)(i - 1) + (size_t)ix * ((size_t)(j - 1) + (size_t)jx * (size_t)(k - 1));
-            const size_t src = (size_t)(per_img(i, ix, mx) - 1) +
-                               (size_t)ix * ((size_t)(per_img(j, jx, my) - 1) + (size_t)jx * (size_t)(per_img(k, kx, mz) - 1));
-            for (int f = 0; f < a.nf; f++) a.q[f][dst] = a.q[f][src];
+            unsigned neg = 0;
+            const int si = map_img(a.map, 0, i, ix, mx, neg), sj = map_img(a.map, 1, j, jx, my, neg),
+                      sk = map_img(a.map, 2, k, kx, mz, neg);
+            const size_t src = (size_t)(si - 1) + (size_t)ix * ((size_t)(sj - 1) + (size_t)jx * (size_t)(sk - 1));
+            double v[NF];
+#pragma unroll
+            for (int f = 0; f < NF; f++) v[f] = a.q[f][src];
+#pragma unroll
+            for (int f = 0; f < NF; f++) a.q[f][dst] = (neg >> f) & 1u ? -v[f] : v[f];
         }
     }
 }
@@ -309,28 +339,60 @@ hipError_t launch_metric(const double *d, const double *dm, int n, Metric m, hip
 hipError_t launch_bnd(const BndArgs &a, hipStream_t s) {
     const int n = a.dir == 0 ? a.ix : (a.dir == 1 ? a.jx : a.kx);
     const long nlines = (long)a.ix * a.jx * a.kx / n;
-    const long total = nlines * a.nf;
-    if (total <= 0) return hipSuccess;
-    hipLaunchKernelGGL(bnd_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s, a);
+    int w = a.margin > 1 ? a.margin : 1;     // at least the thread of a wall's zero (bdsmn with no margin)
+    for (int f = 0; f < a.nf; f++)
+        if (a.kind[f] == BD_PER && a.mbnd > w) w = a.mbnd;
+    const long total = nlines * w;
+    if (total <= 0 || a.nf <= 0) return hipSuccess;
+    const dim3 grid((unsigned)((total + 255) / 256), (unsigned)a.nf);
+    const bool x = a.dir == 0, y = a.dir == 1;
+    const long plane = (long)a.ix * a.jx, minor = x ? w : nlines, fast = y ? a.ix : nlines;
+    const long sfast = x ? a.ix : 1, sslow = y ? plane : 0, stride = x ? 1 : (y ? a.ix : plane);
+    if (total + 255 < (1L << 32)) {
+        const BndLines<unsigned> g{(unsigned)total, (unsigned)minor, x, n, (unsigned)fast, sfast, sslow, stride};
+        hipLaunchKernelGGL(bnd_kernel<unsigned>, grid, dim3(256), 0, s, a, g);
+    } else {
+        const BndLines<unsigned long> g{(unsigned long)total, (unsigned long)minor, x, n, (unsigned long)fast, sfast,
+                                        sslow, stride};
+        hipLaunchKernelGGL(bnd_kernel<unsigned long>, grid, dim3(256), 0, s, a, g);
+    }
     return hipGetLastError();
 }
 
-hipError_t launch_bnd_periodic(double *const *q, int nf, int ix, int jx, int kx, int dim, int m, hipStream_t s) {
+hipError_t launch_bnd_map(double *const *q, int nf, int ix, int jx, int kx, int dim, int m, const BndMap &map,
+                          hipStream_t s) {
     if (nf < 1 || nf > kMaxBndFields || m < 1) return hipErrorInvalidValue;
-    PerFill a{};
+    MapFill a{};
     for (int f = 0; f < nf; f++) a.q[f] = q[f];
-    a.nf = nf; a.ix = ix; a.jx = jx; a.kx = kx;
+    a.ix = ix; a.jx = jx; a.kx = kx;
     a.mx = m; a.my = dim >= 2 ? m : 0; a.mz = dim >= 3 ? m : 0;
-    const int n[3] = {ix, jx, kx}, mm[3] = {a.mx, a.my, a.mz};
-    for (int d = 0; d < 3; d++)
-        if (mm[d] && n[d] - 2 * mm[d] < mm[d]) return hipErrorInvalidValue;   // one shift must reach the interior
+    a.map = map;
+    const int n[3] = {ix, jx, kx};
+    for (int d = 0; d < dim; d++)
+        for (int side = 0; side < 2; side++) {   // the copies must lie in the interior (bnd_map)
+            const int k = map.kind[d][side];
+            if (n[d] - 2 * m < (k == BM_FRE ? 1 : k == BM_SM ? m + 1 : m)) return hipErrorInvalidValue;
+        }
     const long long nchunk = (ix + 63) / 64;
     a.na = (2LL * a.mz * jx + (long long)(kx - 2 * a.mz) * 2 * a.my) * nchunk;
     a.nb = ((long long)(jx - 2 * a.my) * (kx - 2 * a.mz) * 2 * a.mx + 63) / 64;
     long long blocks = (a.na + a.nb + 3) / 4;
     if (blocks > 4096) blocks = 4096;
     if (blocks < 1) return hipSuccess;
-    hipLaunchKernelGGL(per_fill_kernel, dim3((unsigned)blocks), dim3(256), 0, s, a);
+    const bool small = (a.na + a.nb + 4 * blocks + 1) * 64 < (1LL << 32);
+#define FILL(NF)                                                                                                     \
+    case NF:                                                                                                         \
+        if (small) hipLaunchKernelGGL((map_fill_kernel<unsigned, NF>), dim3((unsigned)blocks), dim3(256), 0, s, a);  \
+        else hipLaunchKernelGGL((map_fill_kernel<unsigned long long, NF>), dim3((unsigned)blocks), dim3(256), 0, s, a); \
+        break
+    switch (nf) {   // the field lists of the runs
+        FILL(5);
+        FILL(7);
+        FILL(8);
+        FILL(9);
+    default: return hipErrorInvalidValue;
+    }
+#undef FILL
     return hipGetLastError();
 }
 

@@ -39,6 +39,8 @@ CANS_DEV long long uni(long long v) {
     const unsigned hi = (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)((unsigned long long)v >> 32));
     return (long long)(((unsigned long long)hi << 32) | lo);
 }
+CANS_DEV unsigned uni(unsigned v) { return (unsigned)__builtin_amdgcn_readfirstlane((int)v); }
+CANS_DEV unsigned long long uni(unsigned long long v) { return (unsigned long long)uni((long long)v); }
 
 // Workgroup min of a double (NaN never wins: callers feed only values that
 // passed `v < current`); `red` holds BT/64 doubles.  The result is uniform.
