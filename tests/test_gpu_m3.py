@@ -114,6 +114,57 @@ def test_mlw_m3_2d_resident_loop(oracle, dev, margin, ghost_min):
         assert_bitwise(to_host(g), a[k], k)
 
 
+FRE, SPP, SPN, SMP, SMN, CNS, FRD, PER = range(8)
+BOUNDS = {   # per face (x low, x high, y low, y high): one kind, or nine
+    "mirrors": ([SPP, SPP, SPN, SPP, SPP, SPN, SPP, SPP, SPN], SMP, SMP, [SPP, SPP, SPP, SPN, SPP, SPP, SPN, SPN, SPN]),
+    "free and periodic": (FRE, SMP, PER, PER),
+    "periodic": (PER, PER, PER, PER),
+    # a face with a mixture: cfl_m3, engine and fills one by one
+    "mixed": ([FRE, SPP, FRE, FRE, FRE, SPP, FRE, FRE, FRE], FRE, SMP, FRE),
+}
+
+
+@pytest.mark.parametrize("bounds", list(BOUNDS))
+@pytest.mark.parametrize("nx,ny,margin", [(70, 33, 1), (124, 40, 2), (7, 9, 3), (4, 5, 1)])
+def test_mlw_m3_2d_bounds(oracle, dev, bounds, nx, ny, margin):
+    """Every face kind that the step kernel maps (and a run that it does not),
+    signs per field, smallest spacings in ghost cells, one strip and several;
+    two calls of one run, against cfl_m3, mlw_m3 and the bd* one by one."""
+    print(f"mlw_m3 bounds {bounds} {nx}x{ny} margin {margin}", flush=True)
+    bc = [k for face in BOUNDS[bounds] for k in (face if isinstance(face, list) else [face] * 9)]
+    ix, jx = nx + 2 * margin, ny + 2 * margin
+    s = state2(ix, jx, ix + jx)
+    _, dx, dxm = stretched_grid(ix, seed=ix)
+    _, dy, dym = stretched_grid(jx, seed=jx + 7)
+    dx[0], dx[-1], dy[0], dy[-1] = 0.4 * dx.min(), 0.3 * dx.min(), 0.5 * dy.min(), 0.35 * dy.min()
+    a = {k: v.copy(order="F") for k, v in s.items()}
+    n, dts = 5, []
+    for _ in range(n):
+        dt, merr, _l = oracle.cfl_m3_2d(0.3, 1e-10, 5 / 3, *[a[k] for k in F2[:8]], dx, dy)
+        assert merr == 0
+        oracle.mlw_m3_2d(*[a[k] for k in F2], dt, 3.0, 5 / 3, dx, dxm, dy, dym)
+        for d in (0, 1):
+            for side in (0, 1):
+                for q, k in enumerate(F2):
+                    kind = bc[(2 * d + side) * 9 + q]
+                    if kind == PER:
+                        if side == 0:
+                            oracle.bnd_2d(d, PER, margin, margin, a[k])
+                    else:
+                        oracle.bnd_2d(d, kind, side, margin, a[k], 0.0, dxm if d == 0 else dym)
+        dts.append(dt)
+    grid = {k: T(v, dev) for k, v in dict(dx=dx, dxm=dxm, dy=dy, dym=dym).items()}
+    run = cans.Run(2, cans.ENGINE_MLW3, [to_dev(s[k], dev) for k in F2], grid, 5 / 3, 0.3, qav=3.0, margin=margin,
+                   bc=bc)
+    run.reset(dtmin=1e-10)
+    run.steps(2)
+    run.steps(n - 2)
+    cur, info = run.state()
+    assert info["nexec"] == n and info["dt"] == dts[-1], (info, dts)
+    for k, g in zip(F2, cur):
+        assert_bitwise(to_host(g), a[k], k)
+
+
 def test_mlw_m3_1d_resident_loop(oracle, dev):
     ix, margin, nsteps = 200, 2, 60
     s = state1(ix, 21)

@@ -249,9 +249,9 @@ static int mlw3_dropin(int dim, double *const *f, const double *bx, const double
     if (dim == 2) HIPCHK(launch_metric(dy, dym, jx, m[1], s));
     Mlw3Args a{};
     for (int q = 0; q < nf; q++) { a.in[q] = f[q]; a.out[q] = c.take(N); }
-    a.bx = bx; a.bxm = bxm; a.dxm = dxm; a.dym = dym; a.mx = m[0]; a.my = m[1];
+    a.bx = bx; a.bxm = bxm; a.dx = dx; a.dxm = dxm; a.dy = dy; a.dym = dym; a.mx = m[0]; a.my = m[1];
     a.qav = qav; a.gm = gm; a.dt = dt; a.clk = nullptr; a.ix = ix; a.jx = dim == 2 ? jx : 1;
-    HIPCHK(launch_mlw_m3(a, dim, s));
+    HIPCHK(dim == 1 ? launch_mlw1d_m3(a, s) : launch_mlw2d_m3(a, s));
     const double *src[9];
     for (int q = 0; q < nf; q++) src[q] = a.out[q];
     HIPCHK(launch_copy_interior(f, src, nf, ix, dim == 2 ? jx : 1, 1, 2, s));
@@ -511,8 +511,8 @@ int cans_run(int dim, int engine, int mixed, double *const *a, double *const *b,
     // kernels carry cfl_m and the clock, so a step is the engine and the
     // ghost fill:
     //  * 3D Cartesian MLW (marching kernel), HLLD and FP32-flux Roe (fused z
-    //    marches), 2D mlw_m3: the kernels advance the clock and take the next
-    //    step's cfl_m; the first step of a call still takes cfl_m of its state
+    //    marches): the kernels advance the clock and take the next step's
+    //    cfl_m; 2D mlw_m3 too, with any mapped faces, and writes the ghost cells; the first step of a call still takes cfl_m of its state
     //    in a pass of its own (the same minimum again when the call before
     //    fused it);
     //  * FP64 3D Roe and 2D Roe (roecfl): the stage-1 x faces take the step's
@@ -528,8 +528,8 @@ int cans_run(int dim, int engine, int mixed, double *const *a, double *const *b,
                        (engine == CANS_ENGINE_ROE && (!mixed || roe3d_fused_z(ix, jx, kx))) ||
                        engine == CANS_ENGINE_HLLD);
     const bool roecfl = engine == CANS_ENGINE_ROE && ((per3 && !mixed) || (perio && dim == 2));
-    const bool m3cfl = perio && dim == 2 && m3;
-    const bool fused = per3 || roecfl || m3cfl;
+    const bool m3map = mapped && safety > 0.0 && dim == 2 && m3;
+    const bool fused = per3 || roecfl || m3map;
     for (int st = step0; st < step0 + nsteps; st++) {
         double *const *in = (st & 1) ? b : a;
         double *const *out = (st & 1) ? a : b;
@@ -574,8 +574,15 @@ int cans_run(int dim, int engine, int mixed, double *const *a, double *const *b,
             for (int f = 0; f < nf; f++) { g.in[f] = in[f]; g.out[f] = out[f]; }
             g.bx = bx1d; g.bxm = bxm1d; g.dxm = dxm; g.dym = dym; g.mx = m[0]; g.my = m[1];
             g.qav = qav; g.gm = gm; g.clk = c; g.step = st; g.ix = ix; g.jx = jx;
-            if (m3cfl) { g.dx = dx; g.dy = dy; g.safety = safety; g.per_margin = margin; }
-            HIPCHK(launch_mlw_m3(g, dim, s));
+            if (dim == 1) {
+                HIPCHK(launch_mlw1d_m3(g, s));
+            } else {
+                g.dx = dx; g.dy = dy;
+                // the last step of a call leaves the cfl pass to the next
+                // call, whose caller may change the state in between
+                if (m3map) { g.per_margin = margin; g.safety = st + 1 < step0 + nsteps ? safety : 0.0; }
+                HIPCHK(launch_mlw2d_m3(g, s, m3map && !allper ? &map : nullptr));
+            }
         } else if (sph && dim == 2) {
             Mlw2sArgs g{};
             for (int f = 0; f < 7; f++) { g.prim[f] = in[f]; g.out[f] = out[f]; }
@@ -659,6 +666,7 @@ int cans_run(int dim, int engine, int mixed, double *const *a, double *const *b,
         }
         if (events) HIPCHK(hipEventRecord((hipEvent_t)events[2 * e + 1], s));
         // bnd: x faces, then y, then z; each face: periodic fields both sides
+        if (m3map) continue;
         if (mapped) {
             HIPCHK(launch_bnd_map(out, nf, ix, jx, kx, dim, margin, map, s));
             continue;

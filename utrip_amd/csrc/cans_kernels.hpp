@@ -242,14 +242,17 @@ struct Mlw3Args {
     Clock *clk;                      // non-null: dt and run flag of step `step` (after its clock kernel)
     int step;
     int ix, jx;
-    // 2D mlw_m3 in a periodic box (per_margin = m > 0): the kernel advances
-    // the clock itself and takes the next step's cfl_m3 over the interior
-    // cells it updates (image_min, cfl2_term; dx, dy the cell widths)
+    // 2D mlw_m3 in a run whose ghost cells are copies of interior cells
+    // (per_margin = m > 0): the kernel writes them (a periodic box, or as
+    // launch_mlw2d_m3's map says), advances the clock itself and with safety
+    // > 0 takes the next step's cfl_m3 (cfl2_term).  dx, dy, the cell widths,
+    // are read by every 2D step
     const double *dx, *dy;
     double safety;
     int per_margin;
 };
-hipError_t launch_mlw_m3(const Mlw3Args &a, int dim, hipStream_t s);
+hipError_t launch_mlw1d_m3(const Mlw3Args &a, hipStream_t s);
+hipError_t launch_mlw2d_m3(const Mlw3Args &a, hipStream_t s, const BndMap *map = nullptr);
 // mlw_m_c (cans2d/hdmlw/mlw_m_c.f), fields ro pr vx vz bx bz ay on the (x, z)
 // plane with the radii a.x, a.xm; my is the z metric
 hipError_t launch_mlw_m_c(const Mlw3Args &a, hipStream_t s);
