@@ -321,7 +321,12 @@ class SpiculeRuns:
         L.cans1d_spicule_ws_bytes.restype = C.c_size_t
         nb = L.cans1d_spicule_ws_bytes(C.c_int(ix), C.c_int(n), C.c_int(1 if self.per_run else 0))
         self.ws = torch.empty((nb + 7) // 8, dtype=torch.float64, device=dev)
-        self.block_threads = 256
+        # Threads of a run's workgroup: its 62-cell segments go round its waves
+        # and a run has a CU to itself while there are no more runs than CUs.
+        # 1026 cells, us per step: one run 11.3 with 256 threads, 8.8 with 512;
+        # 1024 runs are fastest with 256 (31 us), which share a CU.
+        cus = torch.cuda.get_device_properties(dev).multi_processor_count
+        self.block_threads = 512 if n <= cus and ix > 4 * 62 + 2 else 256
 
     def run(self, nstop: int = NSTOP, tend: float = TEND, block_threads: Optional[int] = None, blocks: int = 0):
         cans = self._cans
