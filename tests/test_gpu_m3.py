@@ -364,6 +364,22 @@ def test_mlw_m_c_3d_call(oracle, dev, shape):
         assert_bitwise(to_host(d[k]), a[k], k)
 
 
+@pytest.mark.parametrize("shape", [(64, 8, 5), (65, 9, 34), (128, 17, 70)])
+def test_mlw_m_c_3d_tiles(oracle, dev, shape):
+    """Tiles of 63 x 7 corners exactly filled, one over, and several of them
+    in z-segments of more than one plane."""
+    print(f"mlw_m_c 3d tiles {shape}", flush=True)
+    s = smooth_state_3d(*shape, seed=sum(shape) + 1)
+    dx, dxm, dy, dym, dz, dzm = grid3(*shape)
+    x, xm = radii(shape[0], 0.3, dx)
+    a = {k: v.copy(order="F") for k, v in s.items()}
+    oracle.mlw_m_c_3d(*[a[k] for k in F3], 1e-3, 3.0, 5 / 3, x, xm, dx, dxm, dy, dym, dz, dzm)
+    d = {k: to_dev(v, dev) for k, v in s.items()}
+    cans.mlw_m_c_3d(*[d[k] for k in F3], 1e-3, 3.0, 5 / 3, *[T(v, dev) for v in (x, xm, dx, dxm, dy, dym, dz, dzm)])
+    for k in F3:
+        assert_bitwise(to_host(d[k]), a[k], k)
+
+
 def test_mlw_m_c_3d_axis_face_call(oracle, dev):
     shape = (10, 7, 6)
     s = smooth_state_3d(*shape, seed=17)

@@ -56,7 +56,7 @@ size_t engine_doubles(int dim, int engine, size_t N) {
     const size_t a = al(N);
     switch (engine) {
     case CANS_ENGINE_MLW: return dim == 3 ? (size_t)(kMlw3dCellFields + kMlw3dCornerFields) * a : 0;
-    case CANS_ENGINE_MLWC: return dim == 3 ? (size_t)(kMlw3dCylCellFields + kMlw3dCylCornerFields) * a : 0;
+    case CANS_ENGINE_MLWC: return dim == 3 ? (size_t)kMlw3dCylCornerFields * a : 0;
     case CANS_ENGINE_MLWS:
         return (size_t)(dim == 3 ? kMlw3dCylCellFields + kMlw3dCylCornerFields : kMlw2sCellFields + kMlw2sCornerFields) * a;
     case CANS_ENGINE_ROE:
@@ -169,7 +169,7 @@ static int mlw3d_dropin(const char *who, double *const *prim, const double *x, c
     hipStream_t s = (hipStream_t)stream;
     const size_t N = (size_t)ix * jx * kx;
     void *w = nullptr;
-    const int engine = cyl ? CANS_ENGINE_MLWC : CANS_ENGINE_MLW;
+    const int engine = sph ? CANS_ENGINE_MLWS : cyl ? CANS_ENGINE_MLWC : CANS_ENGINE_MLW;
     const size_t need =
         metric_doubles(ix, jx, kx) + engine_doubles(3, engine, N) + 8 * al(N) + (sph ? 6 * al(jx) : 0);
     if (int rc = abi_scratch(need * sizeof(double), &w, s)) return rc;
@@ -181,7 +181,7 @@ static int mlw3d_dropin(const char *who, double *const *prim, const double *x, c
     HIPCHK(launch_metric(dz, dzm, kx, m[2], s));
     Mlw3dArgs a{};
     for (int q = 0; q < 8; q++) a.prim[q] = prim[q];
-    a.cell = c.take((size_t)(cyl ? kMlw3dCylCellFields : kMlw3dCellFields) * al(N));
+    if (sph || !cyl) a.cell = c.take((size_t)(cyl ? kMlw3dCylCellFields : kMlw3dCellFields) * al(N));
     a.corner = c.take((size_t)(cyl ? kMlw3dCylCornerFields : kMlw3dCornerFields) * al(N));
     for (int q = 0; q < 8; q++) a.out[q] = c.take(N);
     a.x = x; a.xm = xm;
@@ -606,7 +606,6 @@ int cans_run(int dim, int engine, int mixed, double *const *a, double *const *b,
             Mlw3dArgs g{};
             for (int q = 0; q < 8; q++) { g.prim[q] = pin[q]; g.out[q] = pout[q]; }
             Carver ec{eng};
-            g.cell = ec.take((size_t)kMlw3dCylCellFields * N);
             g.corner = ec.take((size_t)kMlw3dCylCornerFields * N);
             g.x = bx1d; g.xm = bxm1d;
             g.dxm = dxm; g.dym = dym; g.dzm = dzm; g.mx = m[0]; g.my = m[1]; g.mz = m[2];

@@ -10,16 +10,14 @@
 //            the corner fluxes (mlw_m.f:193-315), 18 values per corner;
 //   update   centre term of mlwhalf, mlwfull.f:34-55, mlwartv.f:36-48,
 //            update and primitive recovery (mlw_m.f:316-453).
-// The same kernels do the curvilinear engines (template G):
-//   G = 1  cylindrical (r, phi, z), cans3d/hdmlw/mlw_m_c.f: phi fluxes divided
-//          by the radius (x at cells, xm at corners) in slots of their own,
-//          and the geometric sources of ro, ee, rx, ry, rz, bz;
-//   G = 2  spherical (r, theta, phi), cans3d/hdmlw/mlw_m_s.f: the conserved
+// The same kernels do the spherical engine (template G; the cylindrical one
+// is in cans_mlw3d_cyl.hip):
+//   G_SPH  spherical (r, theta, phi), cans3d/hdmlw/mlw_m_s.f: the conserved
 //          variables and fluxes carry the metric factors (r^2 sin, r sin, r,
 //          ...), the momenta the geometric sources; the state is unscaled at
 //          the corners and after the update.  sin, cos, tan of the
 //          colatitudes come as per-row tables made on the host.
-// Sources enter at cells into the corner half step (mlwsrch.f:39-46) and the
+// Its sources enter at cells into the corner half step (mlwsrch.f:39-46) and the
 // centre term (mlwsrch.f:33-38), at corners into the update
 // (mlwsrcf.f:33-46).
 #include "cans_common.hpp"
@@ -52,43 +50,6 @@ __constant__ int kCellFlux[8][3][2] = {
     {{C_EZ, -1}, {-1, 1}, {C_EX, 1}},     // by: -ez, 0, ex
     {{C_EY, 1}, {C_EX, -1}, {-1, 1}},     // bz: ey, -ex, 0
 };
-// cylindrical cell slots (mlw_m_c.f:109-243): conserved, x fluxes, raw E,
-// phi fluxes / x, z fluxes, sources
-enum { Y_EEX = 8, Y_RXX, Y_RYX, Y_RZX, Y_EX, Y_EY, Y_EZ,
-       Y_FRO, Y_FEE, Y_FRX, Y_FRY, Y_FRZ, Y_FBX, Y_FBZ,
-       Y_EEZ, Y_RXZ, Y_RYZ, Y_RZZ,
-       Y_SRO, Y_SEE, Y_SRX, Y_SRY, Y_SRZ, Y_SBZ, Y_NCELL };
-static_assert(Y_NCELL == kMlw3dCylCellFields, "cylindrical cell slots");
-// cylindrical corner slots (mlw_m_c.f:273-408)
-enum { Z_ROX, Z_EEX, Z_RXX, Z_RYX, Z_RZX, Z_EX, Z_EY, Z_EZ,
-       Z_FRO, Z_FEE, Z_FRX, Z_FRY, Z_FRZ, Z_FBX, Z_FBZ,
-       Z_ROZ, Z_EEZ, Z_RXZ, Z_RYZ, Z_RZZ,
-       Z_SRO, Z_SEE, Z_SRX, Z_SRY, Z_SRZ, Z_SBZ, Z_NCORN };
-static_assert(Z_NCORN == kMlw3dCylCornerFields, "cylindrical corner slots");
-__constant__ int kCellFluxC[8][3][2] = {
-    {{C_RX, 1}, {Y_FRO, 1}, {C_RZ, 1}},
-    {{Y_EEX, 1}, {Y_FEE, 1}, {Y_EEZ, 1}},
-    {{Y_RXX, 1}, {Y_FRX, 1}, {Y_RXZ, 1}},
-    {{Y_RYX, 1}, {Y_FRY, 1}, {Y_RYZ, 1}},
-    {{Y_RZX, 1}, {Y_FRZ, 1}, {Y_RZZ, 1}},
-    {{-1, 1}, {Y_FBX, 1}, {Y_EY, -1}},    // bx: 0, ez/x, -ey
-    {{Y_EZ, -1}, {-1, 1}, {Y_EX, 1}},     // by: -ez, 0, ex
-    {{Y_EY, 1}, {Y_FBZ, 1}, {-1, 1}},     // bz: ey, -ex/x, 0
-};
-__constant__ int kCornFluxC[8][3][2] = {
-    {{Z_ROX, 1}, {Z_FRO, 1}, {Z_ROZ, 1}},
-    {{Z_EEX, 1}, {Z_FEE, 1}, {Z_EEZ, 1}},
-    {{Z_RXX, 1}, {Z_FRX, 1}, {Z_RXZ, 1}},
-    {{Z_RYX, 1}, {Z_FRY, 1}, {Z_RYZ, 1}},
-    {{Z_RZX, 1}, {Z_FRZ, 1}, {Z_RZZ, 1}},
-    {{-1, 1}, {Z_FBX, 1}, {Z_EY, -1}},
-    {{Z_EZ, -1}, {-1, 1}, {Z_EX, 1}},
-    {{Z_EY, 1}, {Z_FBZ, 1}, {-1, 1}},
-};
-// source slot of each equation (bx, by: none)
-__constant__ int kCellSrc[8] = {Y_SRO, Y_SEE, Y_SRX, Y_SRY, Y_SRZ, -1, -1, Y_SBZ};
-__constant__ int kCornSrc[8] = {Z_SRO, Z_SEE, Z_SRX, Z_SRY, Z_SRZ, -1, -1, Z_SBZ};
-
 // spherical cell slots (mlw_m_s.f:158-321): scaled conserved variables in
 // 0..7, then the scaled x, y, z fluxes and the momentum sources
 enum { P_XRO = 8, P_XEE, P_XRX, P_XRY, P_XRZ, P_XBY, P_XBZ,
@@ -125,9 +86,9 @@ __constant__ int kCornFluxS[8][3][2] = {
 __constant__ int kCellSrcS[8] = {-1, -1, P_SRX, P_SRY, P_SRZ, -1, -1, -1};
 __constant__ int kCornSrcS[8] = {-1, -1, Q_SRX, Q_SRY, Q_SRZ, -1, -1, -1};
 
-enum { G_CART = 0, G_CYL = 1, G_SPH = 2 };
-template <int G> CANS_DEV int csrc(int q) { return G == G_CYL ? kCellSrc[q] : (G == G_SPH ? kCellSrcS[q] : -1); }
-template <int G> CANS_DEV int hsrc(int q) { return G == G_CYL ? kCornSrc[q] : (G == G_SPH ? kCornSrcS[q] : -1); }
+enum { G_CART = 0, G_SPH = 2 };
+template <int G> CANS_DEV int csrc(int q) { return G == G_SPH ? kCellSrcS[q] : -1; }
+template <int G> CANS_DEV int hsrc(int q) { return G == G_SPH ? kCornSrcS[q] : -1; }
 
 __constant__ int kCornFlux[8][3][2] = {
     {{H_ROX, 1}, {H_ROY, 1}, {H_ROZ, 1}},
@@ -232,37 +193,6 @@ __global__ __launch_bounds__(256) void mlw3d_cells(Mlw3dArgs a) {
     const double ey = -vz * bx + vx * bz;
     const double ez = -vx * by + vy * bx;
     const double ep = pr * gm / (gm - 1.0) + 0.5 * ro * vv;
-    if (G == G_CYL) {   // mlw_m_c.f:109-243, r = x(i)
-        const double r = a.x[p % (size_t)a.ix];
-        const double fro = ro * vx;
-        W(Y_FRO, ro * vy / r);
-        W(Y_SRO, -(fro / r));
-        const double fee = ep * vx + (bz * ey - by * ez) * pi4i;
-        W(Y_EEX, fee);
-        W(Y_FEE, (ep * vy + (bx * ez - bz * ex) * pi4i) / r);
-        W(Y_EEZ, ep * vz + (by * ex - bx * ey) * pi4i);
-        W(Y_SEE, -(fee / r));
-        W(Y_RXX, ro * (vx * vx) + pr + pi8i * (by * by + bz * bz - bx * bx));
-        W(Y_FRX, (ro * vx * vy - pi4i * bx * by) / r);
-        W(Y_RXZ, ro * vx * vz - pi4i * bx * bz);
-        W(Y_SRX, -(ro / r * (vx * vx - vy * vy)) + pi4i / r * (bx * bx - by * by));
-        W(Y_RYX, ro * vy * vx - pi4i * by * bx);
-        W(Y_FRY, (ro * (vy * vy) + pr + pi8i * (bx * bx + bz * bz - by * by)) / r);
-        W(Y_RYZ, ro * vy * vz - pi4i * by * bz);
-        W(Y_SRY, -(2.0 * ro / r * vx * vy) + 2.0 * pi4i / r * bx * by);
-        const double frz = ro * vz * vx - pi4i * bz * bx;
-        W(Y_RZX, frz);
-        W(Y_FRZ, (ro * vz * vy - pi4i * bz * by) / r);
-        W(Y_RZZ, ro * (vz * vz) + pr + pi8i * (bx * bx + by * by - bz * bz));
-        W(Y_SRZ, -(frz / r));
-        W(Y_EX, ex);
-        W(Y_EY, ey);
-        W(Y_EZ, ez);
-        W(Y_FBX, ez / r);
-        W(Y_FBZ, -ex / r);
-        W(Y_SBZ, -(ey / r));
-        return;
-    }
     W(C_EEX, ep * vx + (bz * ey - by * ez) * pi4i);
     W(C_EEY, ep * vy + (bx * ez - bz * ex) * pi4i);
     W(C_EEZ, ep * vz + (by * ex - bx * ey) * pi4i);
@@ -283,7 +213,7 @@ __global__ __launch_bounds__(256) void mlw3d_cells(Mlw3dArgs a) {
 
 template <int G>
 CANS_DEV double cflux(const double *c, size_t N, int q, int d, size_t p) {
-    const int(*t)[3][2] = G == G_CYL ? kCellFluxC : (G == G_SPH ? kCellFluxS : kCellFlux);
+    const int(*t)[3][2] = G == G_SPH ? kCellFluxS : kCellFlux;
     const int slot = t[q][d][0];
     if (slot < 0) return 0.0;
     const double v = c[(size_t)slot * N + p];
@@ -291,7 +221,7 @@ CANS_DEV double cflux(const double *c, size_t N, int q, int d, size_t p) {
 }
 template <int G>
 CANS_DEV double hflux(const double *h, size_t N, int q, int d, size_t p) {
-    const int(*t)[3][2] = G == G_CYL ? kCornFluxC : (G == G_SPH ? kCornFluxS : kCornFlux);
+    const int(*t)[3][2] = G == G_SPH ? kCornFluxS : kCornFlux;
     const int slot = t[q][d][0];
     if (slot < 0) return 0.0;
     const double v = h[(size_t)slot * N + p];
@@ -408,39 +338,6 @@ __global__ __launch_bounds__(256) void mlw3d_corners(Mlw3dArgs a) {
         W(Q_ZBY, exh);
         W(Q_XBZ, eyh * r);
         W(Q_YBZ, -exh);
-        return;
-    }
-    if (G == G_CYL) {   // mlw_m_c.f:273-408, r = xm(i)
-        const double r = a.xm[i - 1];
-        const double fro = roh * vxh;
-        W(Z_ROX, fro);
-        W(Z_FRO, roh * vyh / r);
-        W(Z_ROZ, roh * vzh);
-        W(Z_SRO, -(fro / r));
-        const double fee = ep * vxh + (bzh * eyh - byh * ezh) * pi4i;
-        W(Z_EEX, fee);
-        W(Z_FEE, (ep * vyh + (bxh * ezh - bzh * exh) * pi4i) / r);
-        W(Z_EEZ, ep * vzh + (byh * exh - bxh * eyh) * pi4i);
-        W(Z_SEE, -(fee / r));
-        W(Z_RXX, roh * (vxh * vxh) + prh + pi8i * (byh * byh + bzh * bzh - bxh * bxh));
-        W(Z_FRX, (roh * vxh * vyh - pi4i * bxh * byh) / r);
-        W(Z_RXZ, roh * vxh * vzh - pi4i * bxh * bzh);
-        W(Z_SRX, -(roh / r * (vxh * vxh - vyh * vyh)) + pi4i / r * (bxh * bxh - byh * byh));
-        W(Z_RYX, roh * vyh * vxh - pi4i * byh * bxh);
-        W(Z_FRY, (roh * (vyh * vyh) + prh + pi8i * (bxh * bxh + bzh * bzh - byh * byh)) / r);
-        W(Z_RYZ, roh * vyh * vzh - pi4i * byh * bzh);
-        W(Z_SRY, -(2.0 * roh / r * vxh * vyh) + 2.0 * pi4i / r * bxh * byh);
-        const double frz = roh * vzh * vxh - pi4i * bzh * bxh;
-        W(Z_RZX, frz);
-        W(Z_FRZ, (roh * vzh * vyh - pi4i * bzh * byh) / r);
-        W(Z_RZZ, roh * (vzh * vzh) + prh + pi8i * (bxh * bxh + byh * byh - bzh * bzh));
-        W(Z_SRZ, -(frz / r));
-        W(Z_EX, exh);
-        W(Z_EY, eyh);
-        W(Z_EZ, ezh);
-        W(Z_FBX, ezh / r);
-        W(Z_FBZ, -exh / r);
-        W(Z_SBZ, -(eyh / r));
         return;
     }
     W(H_ROX, roh * vxh);
@@ -588,15 +485,12 @@ hipError_t launch_mlw3d(const Mlw3dArgs &a, hipStream_t s) {
     // (a periodic-box call, per_margin > 0, needs the marching kernel: it
     // carries the step's clock and cfl_m)
     if (!a.x && !a.trig && (a.per_margin > 0 || mlw3d_path() == 1)) return launch_mlw3d_march(a, s);
+    if (a.x && !a.trig) return launch_mlw3d_cyl(a, s);
     const dim3 gc(xcd_grid(N)), gk(xcd_grid(nc)), gu(xcd_grid(nu));
     if (a.trig) {
         hipLaunchKernelGGL(mlw3d_cells<G_SPH>, gc, dim3(256), 0, s, a);
         hipLaunchKernelGGL(mlw3d_corners<G_SPH>, gk, dim3(256), 0, s, a);
         hipLaunchKernelGGL(mlw3d_update<G_SPH>, gu, dim3(256), 0, s, a);
-    } else if (a.x) {
-        hipLaunchKernelGGL(mlw3d_cells<G_CYL>, gc, dim3(256), 0, s, a);
-        hipLaunchKernelGGL(mlw3d_corners<G_CYL>, gk, dim3(256), 0, s, a);
-        hipLaunchKernelGGL(mlw3d_update<G_CYL>, gu, dim3(256), 0, s, a);
     } else {
         hipLaunchKernelGGL(mlw3d_cells<G_CART>, gc, dim3(256), 0, s, a);
         hipLaunchKernelGGL(mlw3d_corners<G_CART>, gk, dim3(256), 0, s, a);

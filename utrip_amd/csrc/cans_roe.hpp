@@ -49,7 +49,7 @@ hipError_t launch_roe2d_half(const RoeArgs &a, hipStream_t s);
 struct Mlw3dArgs {
     const double *prim[8];   // ro pr vx vy vz bx by bz (in)
     double *out[8];          // same (out), interior cells
-    double *cell;            // scratch: 23 (curvilinear 32) doubles per cell (SoA)
+    double *cell;            // scratch: 23 (spherical 32) doubles per cell (SoA); cylindrical: none
     double *corner;          // scratch: 18 (curvilinear 26) doubles per corner (SoA)
     const double *x, *xm;    // non-null: curvilinear (mlw_m_c / mlw_m_s), cell and face radii
     const double *trig;      // non-null: spherical mlw_m_s; 6 tables of jx: sin, cos, tan of y, then of ym
@@ -128,5 +128,6 @@ inline int march_segments(size_t cols, int nf) {
 // cans_mlw3d.hip (cans_gpu_set_mlw3d_path changes it).
 int mlw3d_path();
 hipError_t launch_mlw3d_march(const Mlw3dArgs &a, hipStream_t s);
+hipError_t launch_mlw3d_cyl(const Mlw3dArgs &a, hipStream_t s);   // no a.cell
 
 }  // namespace cans
