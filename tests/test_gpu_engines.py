@@ -579,3 +579,52 @@ def test_mixed_precision_3d(dev, oracle, engine):
     print("rel L1 mixed vs fp64:", err)
     assert err["ro"] < 1e-5, err
     assert max(err[k] for k in ("ro", "pr", "bx", "by")) < 1e-4, err
+
+
+@pytest.mark.parametrize("case_", ["mlw 1d", "mlw 2d", "mlw_m3 2d"])
+def test_run_sign_of_density_at_a_face(dev, oracle, case_):
+    """A mirror face that negates ro and pr in its ghost cells: cfl_m sees
+    another Alfven speed there than at the cells they copy, and the ghost
+    spacing is the smallest, so such a run takes cfl_m of every cell."""
+    from tests.test_oracle_m3 import F2 as F2M, state2
+    from utrip_amd import cans
+    case("sign of ro and pr", case_)
+    ix, jx, dim = 40, 30, int(case_[-2])
+    names = F1 if dim == 1 else F2 if case_ == "mlw 2d" else F2M
+    s = smooth_state_1d(ix, seed=3) if dim == 1 else smooth_state_2d(ix, jx, seed=3) if names is F2 else state2(ix, jx, 3)
+    _, dx, dxm = stretched_grid(ix, seed=4)
+    _, dy, dym = stretched_grid(jx, seed=5)
+    dx[0] = 0.2 * dx.min()
+    nf = len(names)
+    bc = [2 if q < 2 else 1 for q in range(nf)] + [0] * nf + ([0] * (2 * nf) if dim == 2 else [])
+    f = {k: v.copy(order="F") for k, v in s.items()}
+    dts = []
+    for _ in range(3):
+        if dim == 1:
+            dt = oracle.cfl_m_1d(0.3, 1e-12, 5 / 3, s["bx"], *[f[k] for k in F1], dx)[0]
+            oracle.mlw_m_1d(*[f[k] for k in F1], s["bx"], s["bxm"], dt, 3.0, 5 / 3, dx, dxm)
+        elif names is F2:
+            dt = oracle.cfl_m_2d(0.3, 1e-12, 5 / 3, *[f[k] for k in F2[:6]], dx, dy)[0]
+            oracle.mlw_m_2d(*[f[k] for k in F2], dt, 3.0, 5 / 3, dx, dxm, dy, dym)
+        else:
+            dt = oracle.cfl_m3_2d(0.3, 1e-12, 5 / 3, *[f[k] for k in F2M[:8]], dx, dy)[0]
+            oracle.mlw_m3_2d(*[f[k] for k in F2M], dt, 3.0, 5 / 3, dx, dxm, dy, dym)
+        dts.append(dt)
+        for d in range(dim):
+            for side in (0, 1):
+                for q, k in enumerate(names):
+                    kind, dm = bc[(2 * d + side) * nf + q], (dxm, dym)[d]
+                    if dim == 1:
+                        oracle.bnd_1d(kind, side, 1, f[k], 0.0, dm)
+                    else:
+                        oracle.bnd_2d(d, kind, side, 1, f[k], 0.0, dm)
+    kw = dict(bx1d=to_dev(s["bx"], dev), bxm1d=to_dev(s["bxm"], dev)) if dim == 1 else {}
+    grid = {k: to_dev(v, dev) for k, v in (dict(dx=dx, dxm=dxm) if dim == 1 else dict(dx=dx, dxm=dxm, dy=dy, dym=dym)).items()}
+    run = cans.Run(dim, cans.ENGINE_MLW3 if names is F2M else cans.ENGINE_MLW, [to_dev(s[k], dev) for k in names], grid,
+                   5 / 3, 0.3, qav=3.0, margin=1, bc=bc, **kw)
+    run.reset(dtmin=1e-12)
+    run.steps(3)
+    cur, info = run.state()
+    assert info["nexec"] == 3 and info["dt"] == dts[-1], (info, dts)
+    for k, t in zip(names, cur):
+        assert_bitwise(to_host(t), f[k], k)

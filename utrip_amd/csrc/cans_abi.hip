@@ -458,7 +458,7 @@ int cans2d_mlw_run(double *const *a7, double *const *b7, void *clk, int step0, i
     // leaves it to the next call: a caller may change the state between calls.
     BndMap map;
     const int nn[2] = {ix, jx};
-    const bool mapped = !periodic && safety > 0.0 && bnd_map(bc, 2, 7, nn, margin, &map);
+    const bool mapped = !periodic && safety > 0.0 && bnd_map(bc, 2, 7, nn, margin, &map) && map.cfl_same(2);
     for (int n = step0; n < step0 + nsteps; n++) {
         double *const *in = (n & 1) ? b7 : a7;
         double *const *out = (n & 1) ? a7 : b7;

@@ -455,7 +455,7 @@ int cans_run(int dim, int engine, int mixed, double *const *a, double *const *b,
     if (engine == CANS_ENGINE_MLW && dim == 2) {   // no bc: the periodic box; one map a face: the same fused kernel
         BndMap map;
         const int nn[2] = {ix, jx};
-        if (!bc || (safety > 0.0 && bnd_map(bc, 2, 7, nn, margin, &map)))
+        if (!bc || (safety > 0.0 && bnd_map(bc, 2, 7, nn, margin, &map) && map.cfl_same(2)))
             return cans2d_mlw_run(a, b, clk, step0, nsteps, qav, gm, safety, dx, dxm, ix, dy, dym, jx, bc, margin,
                                   (double *)ws, events, stream);
     }
@@ -512,9 +512,10 @@ int cans_run(int dim, int engine, int mixed, double *const *a, double *const *b,
     // ghost fill:
     //  * 3D Cartesian MLW (marching kernel), HLLD and FP32-flux Roe (fused z
     //    marches): the kernels advance the clock and take the next step's
-    //    cfl_m; 2D mlw_m3 too, with any mapped faces, and writes the ghost cells; the first step of a call still takes cfl_m of its state
-    //    in a pass of its own (the same minimum again when the call before
-    //    fused it);
+    //    cfl_m; 2D mlw_m3 too, with any mapped faces (cfl_same), and writes
+    //    the ghost cells; the first step of a call still takes cfl_m of its
+    //    state in a pass of its own (the same minimum again when the call
+    //    before fused it);
     //  * FP64 3D Roe and 2D Roe (roecfl): the stage-1 x faces take the step's
     //    own cfl_m and the next kernel advances the clock, after the first
     //    step of a call (whose ghost cells need not be images yet), which
@@ -528,7 +529,7 @@ int cans_run(int dim, int engine, int mixed, double *const *a, double *const *b,
                        (engine == CANS_ENGINE_ROE && (!mixed || roe3d_fused_z(ix, jx, kx))) ||
                        engine == CANS_ENGINE_HLLD);
     const bool roecfl = engine == CANS_ENGINE_ROE && ((per3 && !mixed) || (perio && dim == 2));
-    const bool m3map = mapped && safety > 0.0 && dim == 2 && m3;
+    const bool m3map = mapped && safety > 0.0 && map.cfl_same(2) && dim == 2 && m3;
     const bool fused = per3 || roecfl || m3map;
     for (int st = step0; st < step0 + nsteps; st++) {
         double *const *in = (st & 1) ? b : a;

@@ -93,6 +93,14 @@ enum BndMapKind : int { BM_FRE = 0, BM_SP = 1, BM_SM = 2, BM_PER = 3 };
 struct BndMap {
     int kind[3][2];        // per axis and side, a BndMapKind
     unsigned neg[3][2];    // bit f: field f changes sign there (bdspn*)
+    // whether cfl_m sees at a ghost cell what it sees at the cell it copies:
+    // the vectors' signs enter squared, those of ro and pr (fields 0 and 1 of
+    // every list) do not
+    bool cfl_same(int dim) const {
+        for (int d = 0; d < dim; d++)
+            if ((neg[d][0] | neg[d][1]) & 3u) return false;
+        return true;
+    }
 };
 // The map of a run's boundary list bc (per axis, side and field) on n[0..dim)
 // cells with ghost width m >= 1; false where a face mixes maps, has another
