@@ -37,8 +37,8 @@ __global__ void metric_kernel(const double *d, const double *dm, int n, Metric m
 // periodic line too short for its margins, whose copies read ghosts filled
 // before them: there the thread of i = 1 fills the line in order.  Neighbour
 // threads run along memory: i first for x faces, the line otherwise.  I: the
-// index type, 32 bits where the faces fit (64-bit divisions were most of the
-// kernel).
+// index type, 32 bits where the faces fit (a 512-cell face: a thread per line
+// 4.59 us, per ghost cell 4.08, with 32-bit indices 3.63).
 template <class I>
 struct BndLines {
     I total, minor;          // threads a field; the extent of their faster index (i on x faces, else the line)
