@@ -581,20 +581,21 @@ def test_mixed_precision_3d(dev, oracle, engine):
     assert max(err[k] for k in ("ro", "pr", "bx", "by")) < 1e-4, err
 
 
-@pytest.mark.parametrize("case_", ["mlw 1d", "mlw 2d", "mlw_m3 2d"])
-def test_run_sign_of_density_at_a_face(dev, oracle, case_):
+@pytest.mark.parametrize("case_,margin", [("mlw 1d", 1), ("mlw 1d", 2), ("mlw 1d", 3), ("mlw 2d", 1), ("mlw_m3 2d", 1)])
+def test_run_sign_of_density_at_a_face(dev, oracle, case_, margin):
     """A mirror face that negates ro and pr in its ghost cells: cfl_m sees
     another Alfven speed there than at the cells they copy, and the ghost
-    spacing is the smallest, so such a run takes cfl_m of every cell."""
+    spacing is the smallest (of those cfl_m visits: 1D starts at cell 2, a
+    ghost from margin 2 on), so such a run takes cfl_m of every cell."""
     from tests.test_oracle_m3 import F2 as F2M, state2
     from utrip_amd import cans
-    case("sign of ro and pr", case_)
+    case("sign of ro and pr", case_, "margin", margin)
     ix, jx, dim = 40, 30, int(case_[-2])
     names = F1 if dim == 1 else F2 if case_ == "mlw 2d" else F2M
     s = smooth_state_1d(ix, seed=3) if dim == 1 else smooth_state_2d(ix, jx, seed=3) if names is F2 else state2(ix, jx, 3)
     _, dx, dxm = stretched_grid(ix, seed=4)
     _, dy, dym = stretched_grid(jx, seed=5)
-    dx[0] = 0.2 * dx.min()
+    dx[1 if dim == 1 else 0] = 0.2 * dx.min()
     nf = len(names)
     bc = [2 if q < 2 else 1 for q in range(nf)] + [0] * nf + ([0] * (2 * nf) if dim == 2 else [])
     f = {k: v.copy(order="F") for k, v in s.items()}
@@ -615,13 +616,13 @@ def test_run_sign_of_density_at_a_face(dev, oracle, case_):
                 for q, k in enumerate(names):
                     kind, dm = bc[(2 * d + side) * nf + q], (dxm, dym)[d]
                     if dim == 1:
-                        oracle.bnd_1d(kind, side, 1, f[k], 0.0, dm)
+                        oracle.bnd_1d(kind, side, margin, f[k], 0.0, dm)
                     else:
-                        oracle.bnd_2d(d, kind, side, 1, f[k], 0.0, dm)
+                        oracle.bnd_2d(d, kind, side, margin, f[k], 0.0, dm)
     kw = dict(bx1d=to_dev(s["bx"], dev), bxm1d=to_dev(s["bxm"], dev)) if dim == 1 else {}
     grid = {k: to_dev(v, dev) for k, v in (dict(dx=dx, dxm=dxm) if dim == 1 else dict(dx=dx, dxm=dxm, dy=dy, dym=dym)).items()}
     run = cans.Run(dim, cans.ENGINE_MLW3 if names is F2M else cans.ENGINE_MLW, [to_dev(s[k], dev) for k in names], grid,
-                   5 / 3, 0.3, qav=3.0, margin=1, bc=bc, **kw)
+                   5 / 3, 0.3, qav=3.0, margin=margin, bc=bc, **kw)
     run.reset(dtmin=1e-12)
     run.steps(3)
     cur, info = run.state()

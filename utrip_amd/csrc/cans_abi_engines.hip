@@ -491,8 +491,10 @@ int cans_run(int dim, int engine, int mixed, double *const *a, double *const *b,
     BndMap map;
     const bool mapped = bnd_map(bc, dim, nf, n, margin, &map);
     // 1D MLW so: all the call's steps in one launch (events bracket single
-    // steps, so a call with events takes them one by one)
-    if (engine == CANS_ENGINE_MLW && dim == 1 && mapped && !events && nsteps > 0 && safety > 0.0 && ix <= kRun1dMax) {
+    // steps, so a call with events takes them one by one; the kernel takes a
+    // ghost cell's cfl_m term from the cell it copies: cfl_same)
+    if (engine == CANS_ENGINE_MLW && dim == 1 && mapped && map.cfl_same(1) && !events && nsteps > 0 && safety > 0.0 &&
+        ix <= kRun1dMax) {
         Run1dArgs g{};
         for (int f = 0; f < 5; f++) { g.a[f] = a[f]; g.b[f] = b[f]; }
         g.bx = bx1d; g.bxm = bxm1d; g.dx = dx; g.dxm = dxm; g.di = m[0].di; g.dim = m[0].dim;

@@ -147,7 +147,7 @@ struct BndArgs {
 };
 
 // Steps step0 .. step0+nsteps-1 of one resident 1D MLW run in one launch
-// (cans_run1d.hip); its faces are those of a BndMap.
+// (cans_run1d.hip); its faces are those of a BndMap with cfl_same(1).
 struct Run1dArgs {
     double *a[5], *b[5];                             // buffer sets: ro pr vx vy by
     const double *bx, *bxm, *dx, *dxm, *di, *dim;
