@@ -44,14 +44,35 @@ CANS_DEV unsigned long long uni(unsigned long long v) { return (unsigned long lo
 
 // Workgroup min of a double (NaN never wins: callers feed only values that
 // passed `v < current`); `red` holds BT/64 doubles.  The result is uniform.
+// Two forms, the same value.  With 8 or 16 waves a step waits for the minimum,
+// and the DPP rows are the shorter chain (spicule, one run, us a step: 512
+// threads 8.98 by shuffles, 8.74 by DPP; 1024 threads 9.77, 9.08; resident
+// tube of 1024 cells 5.35, 4.59).  With up to 4 waves several workgroups share
+// a CU and issue counts: DPP moves take VALU slots that the shuffles leave to
+// the others (1024 spicules of 256 threads 32.9 us a step by shuffles, 33.5 by
+// DPP, on another box 32.0 and 33.0; one run 11.05, 11.18; tubes and short
+// resident runs equal).
 template <int BT>
 CANS_DEV double block_min(double v, double *red) {
     constexpr int NW = BT / 64;
-    v = wave_min(v);                       // the same value in every lane
+    static_assert(NW <= 16 && (NW & (NW - 1)) == 0, "waves of a block");
+    if constexpr (NW <= 4) {
+        for (int off = 32; off > 0; off >>= 1) {
+            const double o = __shfl_xor(v, off, 64);
+            v = (o < v) ? o : v;
+        }
+    } else {
+        v = wave_min(v);
+    }
     red[threadIdx.x >> 6] = v;             // all lanes store it: no divergent branch
     __syncthreads();
+    if constexpr (NW <= 4) {
+        double m = red[0];
+#pragma unroll
+        for (int w = 1; w < NW; w++) m = (red[w] < m) ? red[w] : m;
+        return uni(m);
+    }
     // a lane per wave's value, then the row min: no serial chain over NW
-    static_assert(NW <= 16 && (NW & (NW - 1)) == 0, "waves of a block");
     return read_lane(row_min15(red[threadIdx.x & (NW - 1)]), 15);
 }
 
