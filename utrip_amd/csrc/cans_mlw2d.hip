@@ -484,8 +484,8 @@ __global__ __launch_bounds__(WAVE * WPB) __attribute__((amdgpu_waves_per_eu(OCC)
 //
 // Visibility: a wave waits for its stores (vmcnt 0) before the workgroup
 // barrier, wave 0 then adds its units to the step's `done` count with
-// agent-scope release; the last to add acquires, pushes with release, and who
-// takes units acquires before its waves load.
+// agent-scope release; the last to add acquires, pushes with release (the
+// word, then the tail), and who takes units acquires before its waves load.
 enum { B2_UNITS, B2_OWN, B2_START, B2_IDLE, B2_EXIT };
 // A run is shared from this many rounds of its workgroup's waves: at one round
 // the queue costs more than it spreads (1000 runs of 16..64 cells a side 3.0
@@ -493,7 +493,7 @@ enum { B2_UNITS, B2_OWN, B2_START, B2_IDLE, B2_EXIT };
 // 10.9 at three, 15.9 at six; 1024 such runs 37 ms, 71.3 unshared).
 constexpr int kShareRounds = 2;
 constexpr int kShareRuns = 1 << 24;        // run numbers fit a queue word
-constexpr int kShareUnits = 1 << 15;       // units of a step fit, with room for late tickets
+constexpr int kShareUnits = 1 << 15;       // units of a step fit a word
 
 CANS_DEV unsigned long long ald(const unsigned long long *p) {
     return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -534,18 +534,25 @@ CANS_DEV B2Cut batch2d_cut(int ix, int jx, int NW) {
     return c;
 }
 
-// The queue of a group: words (run, units, next ticket) in a ring; [head,
-// tail) are published, resv counts the reserved.
+// The queue of a group: words (run, units, lap, next ticket) in a ring; [head,
+// tail) are published, resv counts the reserved.  The lap of the ring (from 1,
+// mod 64; an empty slot holds 0) says which of a slot's words one is: head and
+// tail are read relaxed, so a ticket might come from what the slot held before
+// the word, and the head must not step over a queued step for that.  1024 runs
+// 36.5 -> 36.9 ms for it; with an acquire before each ticket instead, 37.1.
+constexpr int kTicketBits = 18;            // a step's units (kShareUnits) and the late tickets, 8 a CU
+CANS_DEV unsigned b2_lap(const Batch2dArgs &b, unsigned idx) { return ((idx >> (31 - __builtin_clz(b.cap))) + 1u) & 63u; }
 CANS_DEV void b2_push(const Batch2dArgs &b, int grp, int k, int nunit) {
     Batch2dGroup &g = b.group[grp];
     const unsigned idx = add1(&g.resv, 1u);
     if ((threadIdx.x & 63) == 0)
         __hip_atomic_store(&b.ring[(size_t)grp * b.cap + (idx & (b.cap - 1))],
-                           ((unsigned long long)k << 40) | ((unsigned long long)nunit << 24), __ATOMIC_RELEASE,
-                           __HIP_MEMORY_SCOPE_AGENT);
+                           ((unsigned long long)k << 40) | ((unsigned long long)nunit << 24) |
+                               ((unsigned long long)b2_lap(b, idx) << kTicketBits),
+                           __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
     while ((unsigned)uni((int)ald(&g.tail)) != idx) __builtin_amdgcn_s_sleep(1);
     if ((threadIdx.x & 63) == 0)
-        __hip_atomic_store(&g.tail, idx + 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
+        (void)__hip_atomic_fetch_add(&g.tail, 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
 }
 // What wave 0 found for its workgroup to do: units of its own group's queue,
 // else of another's; a step of the workgroup's own run; the next run.
@@ -563,12 +570,13 @@ CANS_DEV B2Do b2_next(const Batch2dArgs &b, int grp, int NW, bool own) {
         const int g = (grp + __builtin_ctz(turned)) % ng;
         const unsigned hg = (unsigned)__builtin_amdgcn_readlane((int)h, g);
         const unsigned long long w = add1(&b.ring[(size_t)g * b.cap + (hg & (b.cap - 1))], (unsigned long long)NW);
-        const int u = (int)(w & 0xffffffull), n = (int)((w >> 24) & 0xffffull);
+        const int u = (int)(w & ((1ull << kTicketBits) - 1)), n = (int)((w >> 24) & 0xffffull);
         if (u < n) {
             __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
             return B2Do{B2_UNITS, (int)(w >> 40), u, g};
         }
-        if (lane == 0) {   // every unit of the head is taken: the next word
+        const unsigned lap = (unsigned)(w >> kTicketBits) & 63u;
+        if (lane == 0 && lap == b2_lap(b, hg)) {   // every unit of the head is taken: the next word
             unsigned want = hg;
             __hip_atomic_compare_exchange_strong(&b.group[g].head, &want, hg + 1u, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
                                                  __HIP_MEMORY_SCOPE_AGENT);
@@ -760,9 +768,11 @@ __global__ __launch_bounds__(BT) __attribute__((amdgpu_waves_per_eu(kOccBatch)))
 }
 
 // per-run metric of both axes (the arithmetic of the single-run metric
-// kernel) and the queue counter; block r fills run r
+// kernel) by block r for run r; the queue counters, and the rings empty
 __global__ void batch2d_prep(Batch2dArgs b) {
     const int r = blockIdx.x;
+    const size_t nw = (size_t)b.ngroup * b.cap, step = (size_t)gridDim.x * blockDim.x;
+    for (size_t p = (size_t)r * blockDim.x + threadIdx.x; p < nw; p += step) b.ring[p] = 0ull;
     if (r == 0) {
         if (threadIdx.x == 0) *b.next = 0u;
         if ((int)threadIdx.x < b.ngroup) {
@@ -795,7 +805,7 @@ constexpr int kOcc = 2;   // waves per SIMD the register budget is compiled for
 }  // namespace
 
 hipError_t launch_batch2d(const Batch2dArgs &b, int block_threads, int nblocks, hipStream_t s) {
-    hipLaunchKernelGGL(batch2d_prep, dim3(b.nrun > 0 ? b.nrun : 1), dim3(256), 0, s, b);
+    hipLaunchKernelGGL(batch2d_prep, dim3(b.nrun > 64 ? b.nrun : 64), dim3(256), 0, s, b);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess || b.nrun == 0) return e;
     switch (block_threads) {
