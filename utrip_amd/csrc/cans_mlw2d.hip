@@ -477,8 +477,8 @@ __global__ __launch_bounds__(WAVE * WPB) __attribute__((amdgpu_waves_per_eu(OCC)
 // Nothing waits for a workgroup that may not be resident: a unit in a queue
 // is ready to run, units are taken only by running workgroups, and the one
 // that finishes a step's last unit queues the next.  A workgroup with
-// nothing to do polls until there is no shared run left (`active`), which
-// running workgroups bring about.  (The waiting inside a push is for an
+// nothing to do polls until there is no shared run left (`active`, raised
+// before a run is taken from the list), which running workgroups bring about.  (The waiting inside a push is for an
 // earlier push of the group to be published, a few instructions of a running
 // wave.)
 //
@@ -538,8 +538,9 @@ CANS_DEV B2Cut batch2d_cut(int ix, int jx, int NW) {
 // tail) are published, resv counts the reserved.  The lap of the ring (from 1,
 // mod 64; an empty slot holds 0) says which of a slot's words one is: head and
 // tail are read relaxed, so a ticket might come from what the slot held before
-// the word, and the head must not step over a queued step for that.  1024 runs
-// 36.5 -> 36.9 ms for it; with an acquire before each ticket instead, 37.1.
+// the word, and the head must not step over a queued step for that.  (An
+// acquire before each ticket would do as well: 1024 runs 36.5 -> 37.1 ms, with
+// the laps 36.5.)
 constexpr int kTicketBits = 18;            // a step's units (kShareUnits) and the late tickets, 8 a CU
 CANS_DEV unsigned b2_lap(const Batch2dArgs &b, unsigned idx) { return ((idx >> (31 - __builtin_clz(b.cap))) + 1u) & 63u; }
 CANS_DEV void b2_push(const Batch2dArgs &b, int grp, int k, int nunit) {
@@ -586,10 +587,15 @@ CANS_DEV B2Do b2_next(const Batch2dArgs &b, int grp, int NW, bool own) {
     unsigned *active = &b.group[0].active;   // shared runs, and workgroups that may be starting one
     if (uni((int)ald(b.next)) < b.nrun) {
         add1(active, 1u);
+        // released: who sees the list used up (and acquires) sees this start
+        // in `active` too
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
         const int q = (int)add1(b.next, 1u);
         if (q < b.nrun) return B2Do{B2_START, b.order ? uni(b.order[q]) : q, 0, q % ng};
         add1(active, ~0u);
     }
+    if (uni((int)ald(active)) > 0) return B2Do{B2_IDLE, 0, 0, 0};
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
     return B2Do{uni((int)ald(active)) > 0 ? B2_IDLE : B2_EXIT, 0, 0, 0};
 }
 
