@@ -189,6 +189,19 @@ def random_state(ix, seed):
     return {q: np.asfortranarray(v) for q, v in st.items()}
 
 
+def test_runs_set_up_on_host_tensors():
+    """A set of realizations can be made and looked at on host tensors, where
+    there is no GPU; only run() needs one."""
+    from utrip_amd import LIB_GPU
+    if not LIB_GPU.exists():
+        pytest.skip("libcans_gpu.so not built")
+    sp = spicule.setup(400)
+    runs = spicule.SpiculeRuns(sp, [7, 8], device="cpu")
+    assert runs.block_threads == 256 and runs.info(1) == dict(t=0.0, ns=0, merr=0, seed=8)
+    for k in spicule.FIELDS:
+        assert (runs.state(1)[k] == sp.state[k]).all(), k
+
+
 @pytest.mark.parametrize("ix", [4, 65, 300])
 def test_mlw_m_bg_vs_ref(oracle, refsp, ix):
     _, g = random_geometry(ix, ix)

@@ -325,7 +325,8 @@ class SpiculeRuns:
         # and a run has a CU to itself while there are no more runs than CUs.
         # 1026 cells, us per step: one run 11.3 with 256 threads, 8.8 with 512;
         # 1024 runs are fastest with 256 (31 us), which share a CU.
-        cus = torch.cuda.get_device_properties(dev).multi_processor_count
+        # (Host tensors, set up where there is no GPU, have no CUs to share.)
+        cus = torch.cuda.get_device_properties(dev).multi_processor_count if dev.type == "cuda" else 0
         self.block_threads = 512 if n <= cus and ix > 4 * 62 + 2 else 256
 
     def run(self, nstop: int = NSTOP, tend: float = TEND, block_threads: Optional[int] = None, blocks: int = 0):
