@@ -42,10 +42,12 @@ int cans_gpu_init(int device);
 int cans_gpu_sync(void *stream);
 /* Tuning, no counterpart in the reference: the marching face kernels (HLLD
  * y/z sweeps, 3D Roe y/z fluxes) cut each column of faces into segments so
- * that one launch has at least `waves` wavefronts (fewer waves = longer
- * segments; 32768, the default, leaves the number to the library, which
- * takes it from the grid).  Results do not depend on it. */
+ * that one launch has at least `waves` wavefronts (waves >= 1; fewer waves =
+ * longer segments).  Until it is called, and again after
+ * cans_gpu_auto_march_waves, the library takes the number from the grid.
+ * Results do not depend on it. */
 int cans_gpu_set_march_waves(int waves);
+int cans_gpu_auto_march_waves(void);
 /* Tuning, no counterpart in the reference: the Cartesian 3D MLW step
  * (mlw_m 3D) runs as one kernel marching in z with its cell and corner
  * planes in LDS (path 1, the default) or as three kernels over HBM scratch

@@ -73,6 +73,27 @@ def test_tuning_switches_validate_without_a_gpu():
     with pytest.raises(cans.CansError, match="march waves"):
         cans.set_march_waves(0)
     cans.set_march_waves(32768)
+    cans.set_march_waves(None)
+
+
+def test_march_waves_of_a_caller_are_taken_as_they_are():
+    """A number a caller sets is that number, 32768 (the default before the
+    grid's own number) too: at 105 x 103 x 101 it gives single-face segments
+    and so no fused Roe z march, which the grid's own number takes."""
+    from utrip_amd import LIB_GPU, cans
+    if not LIB_GPU.exists():
+        pytest.skip("libcans_gpu.so not built")
+    waves, fused = cans.lib()._ZN4cans11march_wavesEv, cans.lib()._ZN4cans13roe3d_fused_zEiii
+    fused.restype = C.c_bool
+    try:
+        cans.set_march_waves(None)
+        assert fused(105, 103, 101)
+        for n in (1, 32768):
+            cans.set_march_waves(n)
+            assert waves() == n and fused(105, 103, 101) == (n == 1)
+    finally:
+        cans.set_march_waves(None)
+    assert fused(105, 103, 101)
 
 
 def test_python_mirror_rejects_bad_arrays():

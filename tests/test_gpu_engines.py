@@ -408,11 +408,11 @@ def test_run_3d_periodic_ghost_cfl(dev, oracle, engine, margin, axis):
         grid["d" + nm], grid["d" + nm + "m"] = d, dm
     pb = Problem(base.name, base.fields, grid, base.params)
     ref, dts = oracle_loop(oracle, 3, engine, pb.fields, grid, pb.params, 8, 7, margin)
-    cans.set_march_waves(8 if engine == "roe" else 32768)
+    cans.set_march_waves(8 if engine == "roe" else None)
     try:
         got, info = run_gpu(dev, 3, engine, pb.fields, grid, pb.params, 8, 7, margin)
     finally:
-        cans.set_march_waves(32768)
+        cans.set_march_waves(None)
     assert info["nexec"] == 8 and info["merr"] == 0 and info["dt"] == dts[-1]
     for k in F3:
         assert_bitwise(got[k], ref[k], k)
@@ -423,7 +423,7 @@ def test_run_3d_periodic_ghost_cfl(dev, oracle, engine, margin, axis):
         try:
             got32, info32 = run_gpu(dev, 3, engine, pb.fields, grid, pb.params, 8, 7, margin, mixed=True)
         finally:
-            cans.set_march_waves(32768)
+            cans.set_march_waves(None)
         ref32, info_ref32 = run_gpu(dev, 3, engine, pb.fields, grid, pb.params, 8, 7, margin, mixed=True)
         assert info32["nexec"] == 8 and info32["dt"] == info_ref32["dt"]
         for k in F3:
@@ -455,7 +455,7 @@ def test_run_3d_periodic_stops(dev, oracle, engine, margin, mixed):
     st = [to_dev(pb.fields[k], dev) for k in F3]
     gd = {k: to_dev(v, dev) for k, v in pb.grid.items() if k in ("dx", "dxm", "dy", "dym", "dz", "dzm")}
     eng = {"mlw": cans.ENGINE_MLW, "roe": cans.ENGINE_ROE, "hlld": cans.ENGINE_HLLD}[engine]
-    cans.set_march_waves(8 if engine == "roe" else 32768)
+    cans.set_march_waves(8 if engine == "roe" else None)
     try:
         run = cans.Run(3, eng, st, gd, pp["gm"], pp["safety"], qav=pp.get("qav", 3.0), margin=margin, bc=7,
                        mixed=mixed)
@@ -473,7 +473,7 @@ def test_run_3d_periodic_stops(dev, oracle, engine, margin, mixed):
         run.steps(3)
         cur, info = run.state()
     finally:
-        cans.set_march_waves(32768)
+        cans.set_march_waves(None)
     assert info["merr"] == 9001 and info["nexec"] == 0 and info["ns"] == 1
     for k, tt in zip(F3, cur):
         assert_bitwise(to_host(tt), pb.fields[k], k)
@@ -499,11 +499,11 @@ def test_longer_runs_of_the_fused_paths(dev, oracle, dim, engine, n, margin, nst
     ref, dts = oracle_loop(oracle, dim, engine, pb.fields, pb.grid, pb.params, nsteps, 7, margin)
     # 3D: a low wave target, so that the march segments are long (the 3D Roe
     # takes its fused z march on segments of >= 8 faces)
-    cans.set_march_waves(8 if dim == 3 else 32768)
+    cans.set_march_waves(8 if dim == 3 else None)
     try:
         got, info = run_gpu(dev, dim, engine, pb.fields, pb.grid, pb.params, nsteps, 7, margin)
     finally:
-        cans.set_march_waves(32768)
+        cans.set_march_waves(None)
     assert info["nexec"] == nsteps and info["dt"] == dts[-1]
     for k in names:
         assert_bitwise(got[k], ref[k], k)
@@ -525,7 +525,7 @@ def test_run_3d_blast_long_segments(dev, oracle, engine, waves):
         got, info = run_gpu(dev, 3, engine, pb.fields, pb.grid, pb.params, 6, 7, margin)
         got32, _ = run_gpu(dev, 3, engine, pb.fields, pb.grid, pb.params, 6, 7, margin, mixed=True)
     finally:
-        cans.set_march_waves(32768)
+        cans.set_march_waves(None)
     assert info["nexec"] == 6 and info["dt"] == dts[-1]
     for k in F3:
         assert_bitwise(got[k], ref[k], k)
@@ -554,7 +554,7 @@ def test_run_3d_default_segments(dev, engine, mixed, shape):
     try:
         ref, iref = run_gpu(dev, 3, engine, fields, grid, pp, 3, 7, 3, mixed=mixed)
     finally:
-        cans.set_march_waves(32768)
+        cans.set_march_waves(None)
     assert info["nexec"] == 3 and info["dt"] == iref["dt"]
     for k in F3:
         assert_bitwise(got[k], ref[k], k)

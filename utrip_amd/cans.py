@@ -46,12 +46,15 @@ def _check(rc: int) -> None:
         raise CansError(f"libcans_gpu error {rc}: {lib().cans_gpu_last_error().decode()}")
 
 
-def set_march_waves(waves: int) -> None:
+def set_march_waves(waves: Optional[int]) -> None:
     """Minimum wavefronts per launch of the marching face kernels (HLLD y/z
-    sweeps, 3D Roe y/z fluxes): fewer waves, longer segments.  The default,
-    32768, leaves the number to the library (from the grid's sizes).
+    sweeps, 3D Roe y/z fluxes): fewer waves, longer segments.  None, the
+    default, leaves the number to the library (from the grid's sizes).
     Results do not depend on it."""
-    _check(lib().cans_gpu_set_march_waves(int(waves)))
+    if waves is None:
+        _check(lib().cans_gpu_auto_march_waves())
+    else:
+        _check(lib().cans_gpu_set_march_waves(int(waves)))
 
 
 def set_mlw3d_path(path: int) -> None:

@@ -135,6 +135,11 @@ int cans_gpu_set_march_waves(int waves) {
     return 0;
 }
 
+int cans_gpu_auto_march_waves(void) {
+    g_march_waves.store(kMarchWavesAuto);
+    return 0;
+}
+
 int cans_gpu_set_mlw3d_path(int path) {
     if (path != 0 && path != 1) return fail(CANS_ERR_ARG, "mlw3d path %d (0 or 1)", path);
     g_mlw3d_path.store(path);

@@ -98,7 +98,7 @@ hipError_t launch_hlld(const HlldArgs &a, bool mixed, hipStream_t s);
 // column into segments so that a launch has at least this many waves
 // (cans_gpu_set_march_waves; at the default kMarchWavesAuto the number comes
 // from the grid, march_segments).
-constexpr int kMarchWavesAuto = 32768;
+constexpr int kMarchWavesAuto = 0;   // (not a number of waves)
 int march_waves();
 // Segments of a column of nf faces (or cells) when `cols` columns march, a
 // thread each.  Each segment computes one face twice, so segments want to be
