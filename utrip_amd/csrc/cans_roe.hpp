@@ -103,13 +103,16 @@ int march_waves();
 // Segments of a column of nf faces (or cells) when `cols` columns march, a
 // thread each.  Each segment computes one face twice, so segments want to be
 // long; the chip wants waves (2048 run at a time at two per SIMD).  The rule
-// at the default: 16384 waves, but no segment shorter than 8 faces unless the
-// launch then has under 2048 waves.  Whole steps against 32768 waves at every
-// size (n^3, FP64 Roe / FP32-flux HLLD): 96: 529 -> 435 / 443 -> 356 us,
-// 128: 1107 -> 965 / 866 -> 769, 160: 2047 -> 1792 / 1425 -> 1336, 192: 3412
-// -> 2947 / 2387 -> 2240 (4-face segments before: a fifth of the faces
-// twice, and the separate Roe passes); 256: 6832 -> 6742 / 4977 -> 4917, and
-// 320^3 and 64^3 within 1 %.  16384 against 8192 at 256^3: 6742 / 6883.
+// by default: 16384 waves, but no segment shorter than 8 faces unless the
+// launch then has under 2048 waves; and up to 32768 waves, whose last round
+// wastes less, while the segments keep 12 faces.  Whole steps against 32768
+// waves at every size (n^3, FP64 Roe / FP32-flux HLLD, us): 96: 529 -> 435 /
+// 443 -> 356, 128: 1107 -> 965 / 866 -> 769, 160: 2047 -> 1792 / 1425 -> 1336,
+// 192: 3412 -> 2947 / 2387 -> 2240 (4-face segments before: a fifth of the
+// faces twice, and the separate Roe passes); 256: 6065 -> 6034 / 4743 -> 4698.
+// 16384 waves on the large grids too: 288: 8470 / 6590 against 8485 / 6460,
+// 320: 11660 / 9180 against 11510 / 8950, 384: 20050 / 15680 against 19740 /
+// 15320; 8192 at 256: 6271 / 4879.
 inline int march_segments(size_t cols, int nf) {
     const auto seg_for = [cols](unsigned long long waves) { return (waves * 64 + cols - 1) / cols; };
     unsigned long long nseg;
@@ -118,6 +121,9 @@ inline int march_segments(size_t cols, int nf) {
         nseg = seg_for(16384);
         const unsigned long long cap = lng > few ? lng : few;
         if (nseg > cap) nseg = cap;
+        const unsigned long long many = seg_for(32768), twelve = (unsigned long long)nf / 12;
+        const unsigned long long more = many < twelve ? many : twelve;
+        if (nseg < more) nseg = more;
     } else {
         nseg = seg_for((unsigned long long)march_waves());
     }
