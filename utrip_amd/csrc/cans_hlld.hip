@@ -537,7 +537,7 @@ hipError_t launch_hlld_t(const HlldArgs &a, hipStream_t s) {
                 hipLaunchKernelGGL(hlld_sweep_x<T>, dim3((unsigned)((waves + 3) / 4)), dim3(256), 0, s, a, stage, fuse);
             } else {
                 const size_t cols = N / n[dir];
-                int nseg = march_segments(cols, n[dir] - 2);
+                int nseg = march_segments(cols, n[dir] - 2, 0);
                 const int H = (n[dir] - 2 + nseg - 1) / nseg;
                 nseg = (n[dir] - 2 + H - 1) / H;
                 const size_t nt = cols * (size_t)nseg;

@@ -786,6 +786,8 @@ hipError_t launch_roe_t(const RoeArgs &a, hipStream_t s) {
     // march, cut into 3-face segments to fill the chip, was 6 % slower.
     const bool fy2 = D == 2 && !C3 && n[0] >= 3 && n[1] >= 3 &&
                      (size_t)(n[0] - 2) * (size_t)(n[1] - 1) >= ((size_t)1 << 19);
+    // 3D marches: waves up to which they take single faces (march_segments)
+    constexpr unsigned long long kOnes = sizeof(T) == 4 ? 8192 : 3072;
     // 3D: z faces fused with the cell updates (roe_zmarch3) on large grids
     const bool fz3 = D == 3 && roe3d_fused_z(n[0], n[1], n[2]);
     // a periodic run's cfl_m: 3D FP32 fluxes in the fused z marches; 3D FP64
@@ -808,7 +810,7 @@ hipError_t launch_roe_t(const RoeArgs &a, hipStream_t s) {
                 const int nf = stage == 1 ? n[2] - 1 : n[2] - 3;
                 const size_t cols = (size_t)(stage == 1 ? n[0] - 2 : n[0] - 4) *
                                     (size_t)(stage == 1 ? n[1] - 2 : n[1] - 4);
-                int nseg = march_segments(cols, nf);
+                int nseg = march_segments(cols, nf, kOnes);
                 int H = (nf + nseg - 1) / nseg;
                 H = H < 8 ? 8 : H;
                 nseg = (nf + H - 1) / H;
@@ -832,7 +834,7 @@ hipError_t launch_roe_t(const RoeArgs &a, hipStream_t s) {
                 const int od = dir == 1 ? 2 : 1;
                 const size_t cols = (size_t)(stage == 1 ? n[0] - 2 : n[0] - 4) *
                                     (size_t)(stage == 1 ? n[od] - 2 : n[od] - 4);
-                int nseg = march_segments(cols, nf);
+                int nseg = march_segments(cols, nf, kOnes);
                 const int H = (nf + nseg - 1) / nseg;
                 nseg = (nf + H - 1) / H;
                 const size_t threads = cols * (size_t)nseg;
@@ -891,7 +893,7 @@ hipError_t launch_roe_t(const RoeArgs &a, hipStream_t s) {
 bool roe3d_fused_z(int ix, int jx, int kx) {
     if (ix < 3 || jx < 3 || kx < 3) return false;
     const int nf = kx - 1;
-    const int nseg = march_segments((size_t)(ix - 2) * (size_t)(jx - 2), nf);
+    const int nseg = march_segments((size_t)(ix - 2) * (size_t)(jx - 2), nf, 0);
     return (nf + nseg - 1) / nseg >= 8;
 }
 

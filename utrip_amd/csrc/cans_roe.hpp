@@ -113,7 +113,14 @@ int march_waves();
 // 16384 waves on the large grids too: 288: 8470 / 6590 against 8485 / 6460,
 // 320: 11660 / 9180 against 11510 / 8950, 384: 20050 / 15680 against 19740 /
 // 15320; 8192 at 256: 6271 / 4879.
-inline int march_segments(size_t cols, int nf) {
+// Small grids whose single faces make up to `ones` waves take single faces:
+// no face is computed twice (Roe; FP64 / FP32-flux, us, 2-face segments
+// against single ones: 48^3 111 / 104 against 108 / 99, 52^3 128 / 119 against
+// 123 / 108; FP64 to 3072 waves, a round and a half of its two waves per SIMD,
+// 56^3 144 against 152 already; FP32-flux, three per SIMD and less to compute
+// twice, to 8192, 72^3 203 against 197, 64x64x128 254 against 258.  The HLLD
+// cells are better off in twos: 48^3 113 / 99 against 119 / 107).
+inline int march_segments(size_t cols, int nf, unsigned long long ones) {
     const auto seg_for = [cols](unsigned long long waves) { return (waves * 64 + cols - 1) / cols; };
     unsigned long long nseg;
     if (march_waves() == kMarchWavesAuto) {
@@ -124,6 +131,7 @@ inline int march_segments(size_t cols, int nf) {
         const unsigned long long many = seg_for(32768), twelve = (unsigned long long)nf / 12;
         const unsigned long long more = many < twelve ? many : twelve;
         if (nseg < more) nseg = more;
+        if ((unsigned long long)cols * (unsigned long long)nf <= ones * 64) nseg = (unsigned long long)nf;
     } else {
         nseg = seg_for((unsigned long long)march_waves());
     }
