@@ -364,10 +364,12 @@ def test_mlw_m_c_3d_call(oracle, dev, shape):
         assert_bitwise(to_host(d[k]), a[k], k)
 
 
-@pytest.mark.parametrize("shape", [(64, 8, 5), (65, 9, 34), (128, 17, 70)])
+@pytest.mark.parametrize("shape", [(64, 8, 5), (65, 9, 34), (128, 17, 70), (69, 12, 90), (16, 70, 120), (65, 31, 158),
+                                   (8, 70, 200), (17, 40, 250)])
 def test_mlw_m_c_3d_tiles(oracle, dev, shape):
     """Tiles of 63 x 7 corners exactly filled, one over, and several of them
-    in z-segments of more than one plane."""
+    in z-segments of more than one plane, of even and uneven widths; narrow
+    grids, whose tiles are 15 x 31 and 7 x 63, one and several in a row."""
     print(f"mlw_m_c 3d tiles {shape}", flush=True)
     s = smooth_state_3d(*shape, seed=sum(shape) + 1)
     dx, dxm, dy, dym, dz, dzm = grid3(*shape)

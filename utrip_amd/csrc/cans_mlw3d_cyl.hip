@@ -5,7 +5,8 @@
 //
 // Two kernels, the corner values between them in HBM (26 a corner: fluxes,
 // the phi ones divided by the radius, and the geometric sources):
-//   corners  a block of 64 x 8 threads marches an (x, y) tile of cells in z.
+//   corners  a block of 64 x 8 threads (on grids narrow in x 16 x 32 or 8 x 64)
+//            marches an (x, y) tile of cells in z.
 //            Each step turns the primitives of a plane into the 39 cell
 //            values (LDS), and forms the 63 x 7 corners below it from the
 //            cells of the plane and from what its own thread kept of the
@@ -27,7 +28,7 @@ namespace {
 
 constexpr double pi8i = 1.0 / kPi / 8.0;
 constexpr double pi4i = 1.0 / kPi / 4.0;
-constexpr int CTX = 64, CTY = 8, CNT = CTX * CTY;   // cells of a tile plane, threads of a block
+constexpr int CNT = 512;   // cells of a tile plane, CTX x CNT / CTX of them; threads of a block
 
 // corner scratch slots (mlw_m_c.f:273-408): x fluxes, E, phi fluxes / xm, z
 // fluxes, sources
@@ -203,10 +204,16 @@ CANS_DEV bool cyl_dt(const Mlw3dArgs &a, double &dt) {   // after the step's clo
 }
 
 // Corners [k0, k1) of the tile (corner k between the cell planes k and k+1,
-// 0-based).
-__global__ __launch_bounds__(CNT) __attribute__((amdgpu_waves_per_eu(2, 2))) void cyl_corners(Mlw3dArgs a, int tiles_x,
-                                                                                             int ntiles, int nseg,
-                                                                                             int seglen) {
+// 0-based), wx x wy of them a plane: the tiles of a row or column have equal
+// widths, since a last one of a few columns, whose rows are stores of less
+// than 64 bytes, took twice as long as the others (64 columns of 30 x 157
+// corners: 111 -> 50 us; the cell and corner kernels before 52).
+template <int CTX>
+__global__ __launch_bounds__(CNT) __attribute__((amdgpu_waves_per_eu(2, 2))) void cyl_corners(Mlw3dArgs a, int wx, int wy,
+                                                                                             int tiles_x, int ntiles,
+                                                                                             int nseg, int seglen) {
+    constexpr int CTY = CNT / CTX;
+    static_assert(CNT % CTX == 0 && CTY > 1, "tile shape");
     const unsigned per = gridDim.x / kXcds;
     const int item = (int)((blockIdx.x % kXcds) * per + blockIdx.x / kXcds);
     if (item >= ntiles * nseg) return;
@@ -219,10 +226,10 @@ __global__ __launch_bounds__(CNT) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     const int k1 = min(kx - 1, k0 + seglen);
     const double gm = a.gm;
     const int t = threadIdx.x, ti = t % CTX, tj = t / CTX;
-    const int gx = (tile % tiles_x) * (CTX - 1) + ti;   // 0-based cell of this thread
-    const int gy = (tile / tiles_x) * (CTY - 1) + tj;
-    const bool cval = gx < ix && gy < jx;
-    const bool kval = ti < CTX - 1 && tj < CTY - 1 && gx <= ix - 2 && gy <= jx - 2;
+    const int gx = (tile % tiles_x) * wx + ti;   // 0-based cell of this thread
+    const int gy = (tile / tiles_x) * wy + tj;
+    const bool cval = ti <= wx && tj <= wy && gx < ix && gy < jx;
+    const bool kval = ti < wx && tj < wy && gx <= ix - 2 && gy <= jx - 2;
     const size_t N = (size_t)ix * jx * kx, sz = (size_t)ix * jx;
     const size_t p0 = cval ? (size_t)gx + (size_t)ix * gy : 0;
     const double r = cval ? a.x[gx] : 1.0, rm = kval ? a.xm[gx] : 1.0;
@@ -529,23 +536,39 @@ __global__ __launch_bounds__(256) void cyl_update(Mlw3dArgs a) {
 hipError_t launch_mlw3d_cyl(const Mlw3dArgs &a, hipStream_t s) {
     if (a.ix < 3 || a.jx < 3 || a.kx < 3) return hipSuccess;
     if (!a.xm) return hipErrorInvalidValue;
-    const int tiles_x = (a.ix - 1 + CTX - 2) / (CTX - 1), tiles_y = (a.jx - 1 + CTY - 2) / (CTY - 1);
-    const int ntiles = tiles_x * tiles_y, nz = a.kx - 1;
-    // z-segments: a block is alone on its CU (its LDS), so a launch takes
-    // rounds of 256; the number of segments with the fewest planes per CU, one
-    // plane read before a segment's first corner
-    int nseg = 1;
+    // The tile shape and the z-segments: a block is alone on its CU (its LDS),
+    // so a launch takes rounds of 256; the number of segments with the fewest
+    // planes per CU, one plane read before a segment's first corner, and the
+    // shape that needs the fewest then, the widest of equal ones.  Narrow grids
+    // leave most lanes of a wide tile idle: 7 x 189 x 260 cells, a step 489 us
+    // with 64 x 8 tiles, 131 with 8 x 64 (175 with the three kernels).  A plane
+    // of a narrow tile that is a piece of its rows takes a third longer (8 or 16
+    // cells in a row of memory): 202 x 126 x 187, 56 planes of 64 x 8 tiles 1162
+    // us a step, 48 of 8 x 64 1217; 65 x 31 x 158, 8 planes 121, 5 of 16 x 32 113.
+    const int nz = a.kx - 1;
+    int ctx = 0, wx = 0, wy = 0, tiles_x = 0, ntiles = 0, nseg = 1;
     long best = -1;
-    for (int n = 1; n <= 64 && n <= nz; n++) {
-        const int len = (nz + n - 1) / n;
-        const int used = (nz + len - 1) / len;
-        const long cost = (((long)ntiles * used + 256 - 1) / 256) * (len + 1);
-        if (best < 0 || cost < best) { best = cost; nseg = used; }
+    for (int c : {64, 16, 8}) {
+        const int mx = c - 1, my = CNT / c - 1;             // corners of a tile
+        const int tx = (a.ix - 1 + mx - 1) / mx, ty = (a.jx - 1 + my - 1) / my;
+        for (int n = 1; n <= 256 && n <= nz; n++) {
+            const int len = (nz + n - 1) / n;
+            const int used = (nz + len - 1) / len;
+            const long cost = (((long)tx * ty * used + 256 - 1) / 256) * (len + 1) * (c < 64 && tx > 1 ? 4 : 3);
+            if (best >= 0 && cost >= best) continue;
+            best = cost;
+            ctx = c; tiles_x = tx; ntiles = tx * ty; nseg = used;
+            wx = (a.ix - 1 + tx - 1) / tx; wy = (a.jx - 1 + ty - 1) / ty;
+        }
     }
     const int seglen = (nz + nseg - 1) / nseg;
     const long items = (long)ntiles * nseg;
     const unsigned grid = (unsigned)((items + kXcds - 1) / kXcds * kXcds);
-    hipLaunchKernelGGL(cyl_corners, dim3(grid), dim3(CNT), 0, s, a, tiles_x, ntiles, nseg, seglen);
+#define CORNERS(c) hipLaunchKernelGGL(cyl_corners<c>, dim3(grid), dim3(CNT), 0, s, a, wx, wy, tiles_x, ntiles, nseg, seglen)
+    if (ctx == 64) CORNERS(64);
+    else if (ctx == 16) CORNERS(16);
+    else CORNERS(8);
+#undef CORNERS
     if (hipError_t e = hipGetLastError()) return e;
     const size_t nu = (size_t)(a.ix - 2) * (a.jx - 2) * (a.kx - 2);
     hipLaunchKernelGGL(cyl_update, dim3(xcd_grid(nu)), dim3(256), 0, s, a);
