@@ -299,9 +299,9 @@ def blast3d_figures(n: int, steps: int, l1_steps: int = 500, early: int = 100):
 
 def c0_figures(no_cpu: bool = False, reps: int = 5):
     """The c0 workload: one Brio-Wu shock tube (nx = 1024, margin 2, free
-    boundaries, gamma 2, safety 0.4, qav 3) run to t = 0.1 on the device
-    clock (cfl_m, mlw_m, bdfrex launches per step, no host round trip);
-    median of `reps` whole runs after a warm-up run.  The CPU leg runs the
+    boundaries, gamma 2, safety 0.4, qav 3) run to t = 0.1 through cans_run
+    (one launch for all its steps; "launch_per_step" by its old name) and
+    through the batch kernel of one tube ("persistent"); median of `reps` whole runs after a warm-up run.  The CPU leg runs the
     same loop over the reference routines built from source (oracle/_ref,
     libcans1d_ref.so) from C (oracle's orref_loop_1d), one core, median of
     `reps` whole runs."""
@@ -340,7 +340,7 @@ def c0_figures(no_cpu: bool = False, reps: int = 5):
     out = {"cells": 1024, "steps": nsteps, "t": info["t"],
            "launch_per_step": {"ms": med, "us_per_step": med * 1e3 / nsteps,
                                "zone_updates_per_s": 1024 * nsteps / (med / 1e3),
-                               "note": "cans_run: cfl_m, clock, mlw_m and bdfrex launches per step"}}
+                               "note": "cans_run: the call's steps in one launch"}}
     # the same run as one persistent workgroup (the batched-tube kernel with
     # one tube): the whole loop on the device, one barrier per step
     tube = {k: pb.fields[k] for k in ("ro", "pr", "vx", "vy", "by", "bx", "bxm")}

@@ -535,12 +535,13 @@ def test_run_3d_blast_long_segments(dev, oracle, engine, waves):
 
 
 @pytest.mark.parametrize("engine,mixed", [("roe", False), ("roe", True), ("hlld", False), ("hlld", True)])
-@pytest.mark.parametrize("shape", [(99, 97, 95), (131, 60, 41), (21, 19, 120)])
+@pytest.mark.parametrize("shape", [(99, 97, 95), (131, 60, 41), (21, 19, 120), (50, 51, 52), (60, 61, 62)])
 def test_run_3d_default_segments(dev, engine, mixed, shape):
     """The default segments of the 3D marches (the grid's own number: 8-face
-    segments and the fused Roe z march at 99x97x95, 3-face ones at 131x60x41,
-    single faces at 21x19x120) against one face per segment and the separate
-    Roe passes: the same bits."""
+    segments and the fused Roe z march at 99x97x95, single faces at
+    21x19x120, 3-face segments and, FP32-flux Roe, single faces at 131x60x41
+    and 60x61x62, HLLD in twos and Roe in single faces at 50x51x52) against one
+    face per segment and the separate Roe passes: the same bits."""
     from utrip_amd import cans
     case("run 3d default segments", engine, "fp32-flux" if mixed else "fp64", shape)
     n = tuple(k + 6 for k in shape)

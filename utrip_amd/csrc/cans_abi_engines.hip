@@ -501,7 +501,8 @@ int cans_run(int dim, int engine, int mixed, double *const *a, double *const *b,
         g.gm = gm; g.qav = qav; g.safety = safety; g.clk = c;
         g.ix = ix; g.margin = margin;
         for (int side = 0; side < 2; side++) { g.kind[side] = map.kind[0][side]; g.neg[side] = map.neg[0][side]; }
-        for (int st = 0; st < nsteps; st += kRun1dSteps) {   // launches of some 10 ms, others' work comes in between
+        // launches of 8 ms (short tubes) to 70 ms (the longest), others' work comes in between
+        for (int st = 0; st < nsteps; st += kRun1dSteps) {
             g.step0 = step0 + st;
             g.nsteps = nsteps - st < kRun1dSteps ? nsteps - st : kRun1dSteps;
             HIPCHK(launch_run1d(g, s));

@@ -159,7 +159,7 @@ struct Run1dArgs {
 };
 // Longest tube (cells, ghosts included) that runs so: beyond it, one CU's
 // issue costs more per step than a launch per routine across the chip (4000
-// cells 14.4 us a step against 17.1, 8000 cells 26.4 against 17.2).
+// cells 14.1 us a step against 17.1, 8000 cells 26.4 against 17.2).
 constexpr int kRun1dMax = 4800;
 constexpr int kRun1dSteps = 4096;   // steps a launch
 hipError_t launch_run1d(const Run1dArgs &a, hipStream_t s);

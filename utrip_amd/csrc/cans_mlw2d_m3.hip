@@ -17,7 +17,7 @@
 // (half step, centred term, viscosity) and one its corner fluxes.
 //
 // A step with its ghost copies, cfl and clock, periodic boxes, against tiles
-// of 31 x 7 cells through LDS (1.5 cells formed per cell stepped, three
+// of 31 x 7 cells through LDS (1.4 cells formed per cell stepped, three
 // barriers) and a fill pass: 64^2 17.9 -> 11.2 us, 256^2 22.9 -> 17.1, 512^2
 // 39.5 -> 26.9, 1024^2 99 -> 54, 2048^2 378 -> 185; no size was better tiled.
 #include "cans_clock.hpp"

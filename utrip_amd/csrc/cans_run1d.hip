@@ -10,10 +10,11 @@
 // code of the batched tubes), the cell at a face writes its ghost copies, the
 // next step's cfl_m term is taken with the update, and the step's only
 // barrier is the dt minimum.  What bounds it is one CU's FP64 issue (about
-// 450 instructions per segment, 17 segments for 1024 cells on 4 SIMDs) and,
-// for short tubes, the step's one chain of dependent FP64 operations.
-// Measured, us a step, against the launches: 256 cells 15.3 -> 2.9, 1024
-// 16.6 -> 4.6, 2000 16.7 -> 7.6, 4000 17.1 -> 14.4.
+// 480 instructions per segment; 1024 cells, 17 segments on 4 SIMDs: 82 % of
+// the step's 4.4 us) and, up to a segment a SIMD, the step's one chain of
+// dependent FP64 operations (2.0 us).  Measured, us a step, against the
+// launches: 256 cells 15.3 -> 2.7, 1024 16.6 -> 4.4, 2000 16.7 -> 7.4, 4000
+// 17.1 -> 14.1.
 // The two buffers of the state live in LDS, with the six per-cell
 // coefficients beside them while they fit (kCapAll cells), then without
 // (kCapState), so that a step waits on no memory; longer tubes keep the
